@@ -22,7 +22,7 @@
 // dispatched heaviest query blocks first, and the query heads sharing a key head for the same
 // query block are placed on the same XCD (their shared tiles hit its L2).
 //
-// fp32 path: a single-wave VALU kernel (one query row per lane), K/V sub-tiles of 64 keys in LDS.
+// fp32 path: sparse_attn_f32_kernel, fp32 MFMA with the keys of a row group split over the waves.
 //
 // Semantics: FlexAttention with BlockMask.from_kv_blocks(kv_num, kv_idx, block) and
 // mask_mod = (kv <= q) & (kv < n) -- ssa/ssa_kernel.py:33-34,125-126; ssa/gemma_ssa.py:159-162,179.
@@ -71,6 +71,11 @@ __device__ constexpr float fast_bound() {
 // norm of rows 64t..64t+63 at tmax2[bk * ntile + t]. A workgroup bounds its scores with the tiles
 // it attends only, so its choice of path depends on no key it does not read (in particular on no
 // key after its query block).
+
+// fp32 path: number of 16-row groups from which a workgroup takes 32 rows (4 waves) instead of 16
+// (8 waves): 768 groups 51 us with 16 rows against 59, 1024 groups 115 against 111, 4800 groups
+// 1453 against 1351
+constexpr int64_t kF32Rows32 = 1024;
 
 struct AttnParams {
   const char* q;
@@ -312,104 +317,224 @@ __device__ inline float pair_sum(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// fp32 path: one wave per 64 query rows, one row per lane. grid = logical items (no remap).
-__global__ __launch_bounds__(64) void sparse_attn_f32_kernel(AttnParams p) {
-  __shared__ __attribute__((aligned(16))) float Ks[64][64];
-  __shared__ __attribute__((aligned(16))) float Vs[64][64];
-  int64_t L = blockIdx.x;
+// fp32 path: flash attention on v_mfma_f32_16x16x4_f32, operands straight from global memory.
+//
+// A workgroup owns 16 CG query rows; its NW waves share them and split the row's 16-key units
+// (unit u of the list belongs to wave u % NW), each with its own running max and sums, joined
+// through LDS in wave order at the end (the order is fixed: bit-identical results across calls).
+//   S^T = K Q^T: MFMA step (j, e) contracts the dims 16 j + 4 quarter + e, so an operand is
+//     element e of the lane's j-th 16-byte load and a row's 64 dims are read in 64-byte runs.
+//   O^T += V^T P^T: the accumulators of S^T (keys 4 quarter + r of the lane's query) are the B
+//     operand as they stand; the V operand takes dims 4 (lane & 15) + dt for output tile dt, so
+//     one 16-byte load per key serves the four tiles.
+// Nothing is staged in LDS: every K / V element a wave loads feeds CG MFMAs, and the next unit is
+// loaded while the current one is multiplied. The bound is the fp32 matrix rate (64 MFMAs of 32
+// cycles per 16 keys and 32 rows); splitting the keys over the waves is what fills the chip when
+// there are few query rows. Measured (whole call) against one lane per query row on the VALU:
+// 1 head, n 4096, block 64, 10 blocks a row 473 -> 20 us (the host's share of a call is most of
+// it); 3 heads, n 12800, block 128, 34 blocks 3.89 -> 0.38 ms; 8 heads, n 32768 14.4 -> 2.55 ms
+// (106 TFLOP/s; a 8192^3 fp32 library product reaches 154). 64 rows per workgroup are no faster
+// (2.58 ms), 16 waves of 16 rows slower (62 us against 51 at 768 row groups).
+template <int CG, int NW>
+__global__ __launch_bounds__(NW * 64, 2) void sparse_attn_f32_kernel(AttnParams p) {
+  constexpr int ROWS = 16 * CG;
+  constexpr int LD = 68;  // row pitch of the joined partials (floats)
+  __shared__ __attribute__((aligned(16))) float so[NW][ROWS][LD];
+  __shared__ float sm[NW][ROWS], sl[NW][ROWS];
+  const int64_t L0 = logical_id(blockIdx.x, p.group);
+  if (L0 >= p.total) return;
+  int64_t L = L0;
   const int64_t qs = L % p.qsub;
   L /= p.qsub;
-  const int64_t h = L % p.Hq;
-  L /= p.Hq;
+  const int64_t hg = L % p.G;
+  L /= p.G;
+  const int64_t kvh = L % p.Hkv;
+  L /= p.Hkv;
   const int64_t b = L % p.B;
   L /= p.B;
   const int64_t i = p.nbq - 1 - L;
-  const int64_t kvh = h / p.G;
-  const int lane = threadIdx.x;
-  const int64_t q0 = i * p.block + qs * 64;
+  const int64_t h = kvh * p.G + hg;
+  const int64_t q0 = i * p.block + qs * ROWS;
   if (q0 >= p.n) return;
-  const int64_t qmax = q0 + 63 < p.n - 1 ? q0 + 63 : p.n - 1;
-  const int64_t qpos = q0 + lane;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 15, quarter = lane >> 4;
+  const int n32 = (int)p.n, nbq32 = (int)p.nbq, blk32 = (int)p.block, q032 = (int)q0;
+  const int qmax = q032 + ROWS - 1 < n32 - 1 ? q032 + ROWS - 1 : n32 - 1;
 
-  const float* qp = reinterpret_cast<const float*>(p.q) + b * p.qsb + h * p.qsh + qpos * p.qsn;
-  float qv[64], ov[64];
+  f32x4 qf[CG][4];
 #pragma unroll
-  for (int e = 0; e < 64; ++e) {
-    qv[e] = qpos < p.n ? qp[e] : 0.0f;
-    ov[e] = 0.0f;
+  for (int c = 0; c < CG; ++c) {
+    const int64_t qr = q0 + 16 * c + col;
+    const float* qp = reinterpret_cast<const float*>(p.q) + b * p.qsb + h * p.qsh + qr * p.qsn;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      qf[c][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      if (qr < p.n) qf[c][j] = *reinterpret_cast<const f32x4*>(qp + 16 * j + 4 * quarter);
+    }
   }
-  const float* kbase = reinterpret_cast<const float*>(p.k) + b * p.ksb + kvh * p.ksh;
-  const float* vbase = reinterpret_cast<const float*>(p.v) + b * p.vsb + kvh * p.vsh;
+  const float* kbase =
+      reinterpret_cast<const float*>(p.k) + b * p.ksb + kvh * p.ksh + 4 * quarter;
+  const float* vbase = reinterpret_cast<const float*>(p.v) + b * p.vsb + kvh * p.vsh + 4 * col;
+
   const int64_t row = (b * p.Hq + h) * p.nbq + i;
   int cnt = p.kv_num[row];
   if (cnt > p.W) cnt = (int)p.W;
   if (cnt < 0) cnt = 0;
   const int32_t* list = p.kv_idx + row * p.W;
-  const int S = (int)(p.block / 64);
-  float m_run = -INFINITY, l_run = 0.0f;
-  const float c2 = p.scale_log2;
-  for (int t = 0; t < cnt * S; ++t) {
-    const int32_t c = list[t / S];
-    if (c < 0 || (int64_t)c >= p.nbq) continue;
-    const int64_t key0 = (int64_t)c * p.block + (int64_t)(t % S) * 64;
-    if (key0 > qmax || key0 >= p.n) continue;
-    __syncthreads();
-    for (int e = lane; e < 64 * 64; e += 64) {
-      const int kr = e >> 6, kc = e & 63;
-      const bool in = key0 + kr < p.n;
-      Ks[kr][kc] = in ? kbase[(key0 + kr) * p.ksn + kc] : 0.0f;
-      Vs[kr][kc] = in ? vbase[(key0 + kr) * p.vsn + kc] : 0.0f;
-    }
-    __syncthreads();
-    float sv[64];
-    float mx = -INFINITY;
-#pragma unroll
-    for (int j = 0; j < 64; ++j) {
-      float s = 0.0f;
-#pragma unroll
-      for (int e = 0; e < 64; e += 4) {
-        const f32x4 kk = *reinterpret_cast<const f32x4*>(&Ks[j][e]);
-        s = fmaf(qv[e], kk[0], s);
-        s = fmaf(qv[e + 1], kk[1], s);
-        s = fmaf(qv[e + 2], kk[2], s);
-        s = fmaf(qv[e + 3], kk[3], s);
+  const int upb = blk32 / 16;  // units per key block
+  int lbase = 0;
+  int32_t lreg = lane < cnt ? list[lane] : -1;
+  int ce = 0, cs = w - NW;
+  auto next_unit = [&]() -> int {  // first key of this wave's next unit, -1 after the last
+    while (true) {
+      cs += NW;
+      while (cs >= upb) {
+        cs -= upb;
+        ++ce;
       }
-      const int64_t key = key0 + j;
-      if (key > qpos || key >= p.n) s = -INFINITY;
-      sv[j] = s;
-      mx = fmaxf(mx, s);
-    }
-    const float m_new = fmaxf(m_run, mx * c2);
-    if (m_new > m_run) {
-      const float alpha = exp2f(m_run - m_new);
-      l_run *= alpha;
-#pragma unroll
-      for (int e = 0; e < 64; ++e) ov[e] *= alpha;
-      m_run = m_new;
-    }
-    const float m_use = m_run == -INFINITY ? 0.0f : m_run;
-#pragma unroll
-    for (int j = 0; j < 64; ++j) {
-      const float pj = exp2f(fmaf(sv[j], c2, -m_use));
-      l_run += pj;
-#pragma unroll
-      for (int e = 0; e < 64; e += 4) {
-        const f32x4 vv = *reinterpret_cast<const f32x4*>(&Vs[j][e]);
-        ov[e] = fmaf(pj, vv[0], ov[e]);
-        ov[e + 1] = fmaf(pj, vv[1], ov[e + 1]);
-        ov[e + 2] = fmaf(pj, vv[2], ov[e + 2]);
-        ov[e + 3] = fmaf(pj, vv[3], ov[e + 3]);
+      if (ce >= cnt) return -1;
+      if (ce - lbase >= 64) {
+        lbase = ce;
+        lreg = ce + lane < cnt ? list[ce + lane] : -1;
+      }
+      const int c = __builtin_amdgcn_readlane(lreg, ce - lbase);
+      if (c >= 0 && c < nbq32) {
+        const int k0 = c * blk32 + cs * 16;
+        if (k0 <= qmax && k0 < n32) return k0;
       }
     }
+  };
+  // rows past the end re-read row n - 1 (their keys are masked)
+  auto load_k = [&](int key0, f32x4* f) {
+    int kr = key0 + col;
+    if (kr > n32 - 1) kr = n32 - 1;
+    const float* kp = kbase + (int64_t)kr * p.ksn;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) f[j] = *reinterpret_cast<const f32x4*>(kp + 16 * j);
+  };
+  auto load_v = [&](int key0, f32x4* f) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      int kr = key0 + 4 * quarter + r;
+      if (kr > n32 - 1) kr = n32 - 1;
+      f[r] = *reinterpret_cast<const f32x4*>(vbase + (int64_t)kr * p.vsn);
+    }
+  };
+
+  f32x4 oacc[CG][4];
+  float m_run[CG], l_part[CG];
+#pragma unroll
+  for (int c = 0; c < CG; ++c) {
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) oacc[c][dt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    m_run[c] = -INFINITY;
+    l_part[c] = 0.0f;
   }
-  if (qpos < p.n) {
-    const float inv = l_run > 0.0f ? 1.0f / l_run : 0.0f;
-    float* op = reinterpret_cast<float*>(p.o) + b * p.osb + h * p.osh + qpos * p.osn;
+  const float c2 = p.scale_log2;
+  f32x4 kf[4], vf[4], kn[4], vn[4];
+  int key0 = next_unit();
+  if (key0 >= 0) {
+    load_k(key0, kf);
+    load_v(key0, vf);
+  }
+  while (key0 >= 0) {
+    const int key1 = next_unit();
+    if (key1 >= 0) {
+      load_k(key1, kn);
+      load_v(key1, vn);
+    }
+    f32x4 s[CG];
 #pragma unroll
-    for (int e = 0; e < 64; ++e) op[e] = ov[e] * inv;
-    if (p.lse != nullptr)
-      p.lse[(b * p.Hq + h) * p.n + qpos] =
-          l_run > 0.0f ? (m_run + log2f(l_run)) * kLn2 : -INFINITY;
+    for (int c = 0; c < CG; ++c) s[c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int c = 0; c < CG; ++c)
+          s[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[j][e], qf[c][j][e], s[c], 0, 0, 0);
+#pragma unroll
+    for (int c = 0; c < CG; ++c) {
+      const int q_first = q032 + 16 * c;
+      if (key0 + 15 > q_first || key0 + 15 >= n32) {
+        const int lim_q = q_first + col, lim = lim_q < n32 - 1 ? lim_q : n32 - 1;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (key0 + 4 * quarter + r > lim) s[c][r] = -INFINITY;
+      }
+      float mx = fmaxf(fmaxf(s[c][0], s[c][1]), fmaxf(s[c][2], s[c][3]));
+      mx = fmaxf(mx, lane_xor(mx, 16));
+      mx = pair_max(mx);
+      const float m_new = fmaxf(m_run[c], mx * c2);
+      if (__any(m_new > m_run[c])) {
+        const float alpha = m_new > m_run[c] ? exp2f(m_run[c] - m_new) : 1.0f;
+        l_part[c] *= alpha;
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) oacc[c][dt] *= alpha;
+        m_run[c] = m_new;
+      }
+      const float m_use = m_run[c] == -INFINITY ? 0.0f : m_run[c];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        s[c][r] = exp2f(fmaf(s[c][r], c2, -m_use));
+        l_part[c] += s[c][r];
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int c = 0; c < CG; ++c)
+          oacc[c][dt] =
+              __builtin_amdgcn_mfma_f32_16x16x4f32(vf[r][dt], s[c][r], oacc[c][dt], 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      kf[j] = kn[j];
+      vf[j] = vn[j];
+    }
+    key0 = key1;
+  }
+
+  // ---- join the waves' partials ----
+#pragma unroll
+  for (int c = 0; c < CG; ++c) {
+    float l = l_part[c] + lane_xor(l_part[c], 16);
+    l = pair_sum(l);
+    if (quarter == 0) {
+      sm[w][16 * c + col] = m_run[c];
+      sl[w][16 * c + col] = l;
+    }
+#pragma unroll
+    for (int rr = 0; rr < 4; ++rr)
+      *reinterpret_cast<f32x4*>(&so[w][16 * c + col][16 * quarter + 4 * rr]) =
+          f32x4{oacc[c][0][rr], oacc[c][1][rr], oacc[c][2][rr], oacc[c][3][rr]};
+  }
+  __syncthreads();
+  for (int t = tid; t < ROWS * 16; t += NW * 64) {
+    const int r = t >> 4, e = (t & 15) * 4;
+    const int64_t qr = q0 + r;
+    if (qr >= p.n) continue;
+    float m = -INFINITY;
+#pragma unroll
+    for (int u = 0; u < NW; ++u) m = fmaxf(m, sm[u][r]);
+    const float m_use = m == -INFINITY ? 0.0f : m;
+    f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
+    float l = 0.0f;
+#pragma unroll
+    for (int u = 0; u < NW; ++u) {
+      const float f = exp2f(sm[u][r] - m_use);
+      l = fmaf(sl[u][r], f, l);
+      const f32x4 x = *reinterpret_cast<const f32x4*>(&so[u][r][e]);
+#pragma unroll
+      for (int a = 0; a < 4; ++a) o[a] = fmaf(x[a], f, o[a]);
+    }
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    float* op = reinterpret_cast<float*>(p.o) + b * p.osb + h * p.osh + qr * p.osn;
+    *reinterpret_cast<f32x4*>(op + e) = o * inv;
+    if (p.lse != nullptr && (t & 15) == 0)
+      p.lse[(b * p.Hq + h) * p.n + qr] = l > 0.0f ? (m + log2f(l)) * kLn2 : -INFINITY;
   }
 }
 
@@ -1469,11 +1594,14 @@ extern "C" int ssa_sparse_attn_fwd(const void* q, const void* k, const void* v, 
   p.ntile = p.n_pad / 64;
   if (dtype == SSA_F32) {
     p.vt = nullptr;
-    p.qsub = block / 64;
-    p.group = 1;
-    p.total = p.nbq * B * Hq * p.qsub;
-    SSA_REQUIRE(p.total < (1ll << 31), SSA_ERR_UNSUPPORTED, "sparse_attn: grid too large");
-    sparse_attn_f32_kernel<<<(unsigned)p.total, 64, 0, st>>>(p);
+    const int cg = p.nbq * B * Hq * (block / 16) >= kF32Rows32 ? 2 : 1;
+    p.qsub = block / (16 * cg);
+    p.group = p.G * p.qsub;
+    p.total = p.nbq * B * Hkv * p.group;
+    const int64_t grid = (p.total + 8 * p.group - 1) / (8 * p.group) * (8 * p.group);
+    SSA_REQUIRE(grid < (1ll << 31), SSA_ERR_UNSUPPORTED, "sparse_attn: grid too large");
+    if (cg == 2) sparse_attn_f32_kernel<2, 4><<<(unsigned)grid, 256, 0, st>>>(p);
+    else sparse_attn_f32_kernel<1, 8><<<(unsigned)grid, 512, 0, st>>>(p);
     return launch_status("sparse_attn_f32_kernel");
   }
   const size_t need = ssa_sparse_attn_workspace_size(dtype, B, Hkv, n, d, block);

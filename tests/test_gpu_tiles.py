@@ -1,0 +1,50 @@
+"""GPU kernels at the sizes where their tilings change or leave remainders, against the CPU oracle
+(float64)."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import ssa_oracle as O
+from ssa_amd import ssa_kernel as K
+from ssa_amd import workloads as WL
+
+pytestmark = pytest.mark.gpu
+
+
+def np_of(t):
+    return t.detach().float().cpu().numpy()
+
+
+def random_lists(rng, rows, nb, W):
+    """Ascending block lists of 1 to min(W, i + 2) blocks (a later block may be among them)."""
+    kv_num = np.zeros((1, rows, nb), np.int32)
+    kv_idx = np.zeros((1, rows, nb, W), np.int32)
+    for h in range(rows):
+        for i in range(nb):
+            m = int(rng.integers(1, min(W, i + 2, nb) + 1))
+            ids = np.sort(rng.permutation(min(i + 2, nb))[:m])
+            kv_num[0, h, i], kv_idx[0, h, i, :m] = m, ids
+    return kv_num, kv_idx
+
+
+# 16-row groups (fewer than 1024) and 32-row groups; a single row; a part of a unit; lists longer
+# than the 64-entry register window
+@pytest.mark.parametrize("hq,hkv,n,block,W", [(1, 1, 1, 64, 2), (2, 1, 79, 64, 3),
+                                              (3, 1, 700, 128, 4), (1, 1, 4608, 64, 72),
+                                              (8, 2, 2075, 64, 6), (6, 6, 3000, 384, 5)])
+def test_fp32_attention_tiles_match_oracle(cuda, hq, hkv, n, block, W):
+    """1e-5: the bar of every fp32 attention test (64-term fp32 dots of N(0,1) at scale 1/8)."""
+    rng = np.random.default_rng(n)
+    q, k, v = (rng.standard_normal((1, h, n, 64)).astype(np.float32) for h in (hq, hkv, hkv))
+    nb = -(-n // block)
+    kv_num, kv_idx = random_lists(rng, hq, nb, min(W, nb))
+    out, lse = K.sparse_attention(*(torch.from_numpy(x).to(cuda) for x in (q, k, v)),
+                                  torch.from_numpy(kv_num).to(cuda),
+                                  torch.from_numpy(kv_idx).to(cuda), block, return_lse=True)
+    ref = O.sparse_attention(q, k, v, kv_num, kv_idx, block)
+    assert np.abs(np_of(out) - ref).max() < 1e-5
+    h, i = hq - 1, nb - 1  # lse of the last row
+    js = [j for c in kv_idx[0, h, i, :kv_num[0, h, i]] for j in range(c * block,
+                                                                       min(n, (c + 1) * block))]
+    s = k[0, h // (hq // hkv), js].astype(np.float64) @ q[0, h, n - 1].astype(np.float64) / 8
+    assert abs(float(lse[0, h, n - 1]) - np.log(np.exp(s).sum())) < 1e-5
