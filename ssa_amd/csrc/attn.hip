@@ -848,8 +848,10 @@ __global__ __launch_bounds__(NW * 64, WPE) void sparse_attn_dma_kernel(AttnParam
   // sub-tiles reuse it as the offset of P = 2^(s - m) (bf16 P has fp32's exponent range, so a
   // later score may exceed m by up to ~100 log2 units before anything overflows). A workgroup
   // with a row whose sum or output left that range walks its list again with the per-sub-tile
-  // running max (xo_pass false).
-  constexpr bool XO = !fast && DT == SSA_BF16;
+  // running max (xo_pass false). Head dim 64 only: at 128 / 256 the body expanded four times left
+  // the accumulators in scratch memory (640 / 1024 bytes a lane) -- 16 heads, n 8192, block 256,
+  // budget 0.25, bf16: d 128 1198 us with it, 109 without; d 256 4271 against 335.
+  constexpr bool XO = !fast && DT == SSA_BF16 && D == 64;
   // raised wave priority around the exact path's MFMA phases: kept for head dims 128 / 256; at 64
   // the default priority is 1.5-2 % faster since the max is no longer taken every sub-tile
   constexpr bool PRIO = !fast && D != 64;
