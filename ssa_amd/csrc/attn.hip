@@ -76,6 +76,13 @@ __device__ constexpr float fast_bound() {
 // (8 waves): 768 groups 51 us with 16 rows against 59, 1024 groups 115 against 111, 4800 groups
 // 1453 against 1351
 constexpr int64_t kF32Rows32 = 1024;
+// head dim 512: number of 128-row groups from which sparse_attn_wide16_kernel runs (8 waves, or 4
+// where a query block holds fewer than 128 rows or the 8-wave grid leaves CUs idle), instead of
+// the 32-row sparse_attn_wide_kernel. Call times at block 256 / 128, budget 0.25, 32-row kernel
+// (+ its V^T pass) / 4 waves / 8 waves: 8 groups 28 (+4) / 37 / 43 us; 64 groups 80 (+5) / 94 /
+// 103; 128 groups 81 (+6) / 73 / 82; 192 groups 139 (+8) / 113 / 102; 448 groups 365 (+14) / 273 /
+// 177; 1024 groups 1359 (+26) / 1020 / 658; block 64, 1024 groups 1072 / 780.
+constexpr int64_t kWide16Min = 96, kWide16Full = 160;
 
 struct AttnParams {
   const char* q;
@@ -1158,6 +1165,257 @@ __global__ __launch_bounds__(NW * 64, WPE) void sparse_attn_dma_kernel(AttnParam
   }
 }
 
+// Head dim 512: the rows' O accumulators decide the tiling. 32 rows of O are 256
+// registers a lane, so a wave owns 16 query rows (128 of O, 64 of Q, two waves per SIMD) and a
+// workgroup of 8 waves 128 rows of a query block, walking the row's selected key blocks in 32-key
+// sub-tiles of K and V (32 KB each) that go HBM -> LDS directly into a 2-stage ring (128 KB).
+//   S^T = K Q^T and O^T += V^T P^T on v_mfma_f32_16x16x32: row m of score tile t takes key
+//     8 (m >> 2) + 4 t + (m & 3), so a lane's eight scores are the eight consecutive keys of its
+//     B operand in the second product and P never leaves registers.
+// V is read as it is and transposed by the LDS reads (ds_read_b64_tr_b16): no V^T pass.
+// Exact path only: running max (lazy rescale), fp32-scaled scores. What bounds it: each wave reads
+// the whole 64 KB sub-tile from LDS for its 16 rows, 4096 LDS cycles a sub-tile against 2048 of
+// MFMA; without any global load the walk takes 80 % of its time. Measured (16 heads, n 8192, block
+// 256, budget 0.25, bf16): 1359 us as 32-row workgroups with the head dim split over the waves
+// (64 KB from L2 for every 32 rows), 658 us here (565 TFLOP/s); 643 us reading a V^T that takes
+// another 26 us to write.
+template <int DT>
+struct Mfma16;
+template <>
+struct Mfma16<SSA_BF16> {
+  static __device__ inline f32x4 mma(const bf16x8& a, const bf16x8& b, const f32x4& c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+  }
+};
+template <>
+struct Mfma16<SSA_F16> {
+  static __device__ inline f32x4 mma(const f16x8& a, const f16x8& b, const f32x4& c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+  }
+};
+
+__device__ inline int kswz(int r) { return (r & 3) | ((r >> 1) & 12); }
+__device__ inline int vswz(int r) { return (r & 3) | ((r >> 1) & 4); }
+
+// Transposing LDS read (ds_read_b64_tr_b16): of the 16 lanes of a group, lane l gives the address
+// of four 16-bit values (its 8 bytes) and receives value l & 3 of lanes 4 j + (l >> 2), j = 0..3:
+// with lane l at row l >> 2, columns 4 (l & 3).. of a 4 x 16 block, column l of the block.
+__device__ inline uint2 lds_read_tr(const unsigned char* p) {
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) s16x4* lds_ptr;
+  return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(p)));
+}
+
+template <int DT, int NW>
+__global__ __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) void sparse_attn_wide16_kernel(AttnParams p) {
+  using M = Mfma<DT>;
+  using M16 = Mfma16<DT>;
+  typedef typename M::vec vec;
+  constexpr int D = 512, KT = 32, ROWS = 16 * NW;
+  constexpr int KD = D / 32;         // k-steps of the QK product
+  constexpr int DTN = D / 16;        // 16-dim output tiles
+  constexpr int TILE = KT * D * 2;   // bytes of a K or V sub-tile
+  constexpr int LPW = TILE / 1024 / NW;
+  __shared__ __attribute__((aligned(1024))) unsigned char kst0[TILE];
+  __shared__ __attribute__((aligned(1024))) unsigned char vst0[TILE];
+  __shared__ __attribute__((aligned(1024))) unsigned char kst1[TILE];
+  __shared__ __attribute__((aligned(1024))) unsigned char vst1[TILE];
+
+  const int64_t L0 = logical_id(blockIdx.x, p.group);
+  if (L0 >= p.total) return;
+  int64_t L = L0;
+  const int64_t qs = L % p.qsub;
+  L /= p.qsub;
+  const int64_t hg = L % p.G;
+  L /= p.G;
+  const int64_t kvh = L % p.Hkv;
+  L /= p.Hkv;
+  const int64_t b = L % p.B;
+  L /= p.B;
+  const int64_t i = p.nbq - 1 - L;
+  const int64_t h = kvh * p.G + hg;
+  const int64_t q0 = i * p.block + qs * ROWS;
+  if (q0 >= p.n) return;
+  const int64_t qmax = q0 + ROWS - 1 < p.n - 1 ? q0 + ROWS - 1 : p.n - 1;
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int quarter = lane >> 4, col = lane & 15;
+  const int n32 = (int)p.n, blk32 = (int)p.block, nbq32 = (int)p.nbq, qmax32 = (int)qmax;
+  const int qw0 = (int)q0 + 16 * w;  // this wave's first query row
+  const int qpos = qw0 + col;
+  const int64_t row = (b * p.Hq + h) * p.nbq + i;
+  int cnt = p.kv_num[row];
+  if (cnt > p.W) cnt = (int)p.W;
+  if (cnt < 0) cnt = 0;
+  const int32_t* list = p.kv_idx + row * p.W;
+  const int S = blk32 / KT;
+
+  vec qf[KD];
+  {
+    const unsigned short* src = reinterpret_cast<const unsigned short*>(p.q) + b * p.qsb +
+                                h * p.qsh + (int64_t)qpos * p.qsn + quarter * 8;
+#pragma unroll
+    for (int kd = 0; kd < KD; ++kd) {
+      u32x4 wv = {0u, 0u, 0u, 0u};
+      if (qpos <= qmax32) wv = *reinterpret_cast<const u32x4*>(src + kd * 32);
+      qf[kd] = M::from_bits(wv);
+    }
+  }
+  const unsigned short* kbase =
+      reinterpret_cast<const unsigned short*>(p.k) + b * p.ksb + kvh * p.ksh;
+  const unsigned short* vbase =
+      reinterpret_cast<const unsigned short*>(p.v) + b * p.vsb + kvh * p.vsh;
+
+  // Load plan: instruction j of wave w fills rows j NW + w of K and V (1 KB: 64 chunks of 16 bytes).
+  // Chunk c of row r is stored at c ^ kswz(r) / c ^ 2 vswz(r): the 16 lanes of one ds_read_b128
+  // phase (K rows 8 a + b + 4 t, a and b in 0..3) hit all 64 banks once, and so do the 32 of a
+  // transposing read (32-byte pieces of V rows 8 a + b, a in {0, 1} or {2, 3}).
+  auto issue = [&](unsigned char* kdst, unsigned char* vdst, int key0) {
+#pragma unroll
+    for (int j = 0; j < LPW; ++j) {
+      const int r = j * NW + w;
+      int kr = key0 + r;
+      if (kr > n32 - 1) kr = n32 - 1;  // ragged tail: re-read row n - 1 (masked below)
+      __builtin_amdgcn_global_load_lds(kbase + (int64_t)kr * p.ksn + ((lane ^ kswz(r)) * 8),
+                                       kdst + r * 1024, 16, 0, 0);
+    }
+#pragma unroll
+    for (int j = 0; j < LPW; ++j) {
+      const int r = j * NW + w;
+      int kr = key0 + r;
+      if (kr > n32 - 1) kr = n32 - 1;
+      __builtin_amdgcn_global_load_lds(vbase + (int64_t)kr * p.vsn + ((lane ^ (2 * vswz(r))) * 8),
+                                       vdst + r * 1024, 16, 0, 0);
+    }
+  };
+
+  int lbase = 0;
+  int32_t lreg = lane < cnt ? list[lane] : -1;
+  int ce = 0, cs = -1;
+  auto next_tile = [&]() -> int {
+    while (true) {
+      if (++cs == S) {
+        cs = 0;
+        ++ce;
+      }
+      if (ce >= cnt) return -1;
+      if (ce - lbase >= 64) {  // wave-uniform; once per 64 list entries
+        lbase = ce;
+        lreg = ce + lane < cnt ? list[ce + lane] : -1;
+      }
+      const int c = __builtin_amdgcn_readlane(lreg, ce - lbase);
+      if (c >= 0 && c < nbq32) {
+        const int k0 = c * blk32 + cs * KT;
+        if (k0 <= qmax32 && k0 < n32) return k0;
+      }
+      cs = S - 1;
+    }
+  };
+
+  // LDS read offsets: K tile t row 8 (col >> 2) + 4 t + (col & 3), chunk 4 kd + quarter (four
+  // k-steps are 256 bytes, past the swizzled bits)
+  const int kr0 = 8 * (col >> 2) + (col & 3);
+  uint32_t koff[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s)
+    koff[s] = (uint32_t)(kr0 * 1024 + (((4 * s + quarter) ^ kswz(kr0)) * 16));
+  // V (transposing reads): keys 8 quarter + 4 hh + (col >> 2), dims 16 dt + 4 (col & 3) .. + 3;
+  // eight output tiles are 256 bytes
+  uint32_t voff[8];
+#pragma unroll
+  for (int u = 0; u < 8; ++u) {
+    const int r = 8 * quarter + (col >> 2);
+    voff[u] = (uint32_t)(r * 1024 + ((u ^ vswz(r)) * 32) + (col & 3) * 8);
+  }
+
+  f32x4 oacc[DTN];
+#pragma unroll
+  for (int dt = 0; dt < DTN; ++dt) oacc[dt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  float m_run = -INFINITY, l_part = 0.0f;
+  const float c2 = p.scale_log2;
+  const int wlast = qw0 + 15 < qmax32 ? qw0 + 15 : qmax32;
+  auto compute = [&](const unsigned char* ks, const unsigned char* vs, int key0) {
+    f32x4 s[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+#pragma unroll
+    for (int kd = 0; kd < KD; ++kd)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const u32x4 a = *reinterpret_cast<const u32x4*>(ks + koff[kd & 3] + (kd >> 2) * 256 +
+                                                        t * 4096);
+        s[t] = M16::mma(M::from_bits(a), qf[kd], s[t]);
+      }
+    float sv[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) sv[j] = s[j >> 2][j & 3];
+    if (key0 + KT - 1 > qw0 || key0 + KT > n32) {  // diagonal / ragged tail sub-tiles
+      const int lim_q = qpos - key0, lim_n = n32 - 1 - key0;
+      const int lim = lim_q < lim_n ? lim_q : lim_n;
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (8 * quarter + j > lim) sv[j] = -INFINITY;
+    }
+    float mx = sv[0];
+#pragma unroll
+    for (int j = 1; j < 8; ++j) mx = fmaxf(mx, sv[j]);
+    mx = fmaxf(mx, lane_xor(mx, 16));
+    mx = pair_max(mx);
+    const float m_cand = mx * c2;
+    const bool grew = m_cand > m_run + kRescaleSlack;
+    if (__any(grew)) {
+      const float alpha = grew ? __builtin_amdgcn_exp2f(m_run - m_cand) : 1.0f;
+      l_part *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < DTN; ++dt) oacc[dt] *= alpha;
+      m_run = grew ? m_cand : m_run;
+    }
+    const float m_use = m_run == -INFINITY ? 0.0f : m_run;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) sv[j] = __builtin_amdgcn_exp2f(fmaf(sv[j], c2, -m_use));
+    const vec pb = M::pack(sv);
+    l_part = M::rowsum(pb, l_part);
+#pragma unroll
+    for (int dt = 0; dt < DTN; ++dt) {
+      const unsigned char* vp = vs + voff[dt & 7] + (dt >> 3) * 256;
+      const uint2 lo = lds_read_tr(vp), hi = lds_read_tr(vp + 4096);
+      oacc[dt] = M16::mma(M::from_bits(u32x4{lo.x, lo.y, hi.x, hi.y}), pb, oacc[dt]);
+    }
+  };
+  int key0 = next_tile();
+  if (key0 >= 0) issue(kst0, vst0, key0);
+  while (key0 >= 0) {
+    int key0n = next_tile();
+    dma_barrier();  // stage 0 landed for all waves; stage 1 no longer read
+    if (key0n >= 0) issue(kst1, vst1, key0n);
+    if (key0 <= wlast) compute(kst0, vst0, key0);
+    key0 = key0n;
+    if (key0 < 0) break;
+    key0n = next_tile();
+    dma_barrier();  // stage 1 landed; stage 0 no longer read
+    if (key0n >= 0) issue(kst0, vst0, key0n);
+    if (key0 <= wlast) compute(kst1, vst1, key0);
+    key0 = key0n;
+  }
+
+  // ---- epilogue: O = O^T / l; the lane's dims 16 dt + 4 quarter .. + 3 ----
+  float l_tot = l_part + lane_xor(l_part, 16);
+  l_tot = pair_sum(l_tot);
+  const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
+  if (qpos <= qmax32) {
+    unsigned short* op = reinterpret_cast<unsigned short*>(p.o) + b * p.osb + h * p.osh +
+                         (int64_t)qpos * p.osn + 4 * quarter;
+#pragma unroll
+    for (int dt = 0; dt < DTN; ++dt) {
+      uint2 wv;
+      wv.x = M::pack2(oacc[dt][0] * inv, oacc[dt][1] * inv);
+      wv.y = M::pack2(oacc[dt][2] * inv, oacc[dt][3] * inv);
+      *reinterpret_cast<uint2*>(op + dt * 16) = wv;
+    }
+    if (p.lse != nullptr && quarter == 0)
+      p.lse[(b * p.Hq + h) * p.n + qpos] = l_tot > 0.0f ? (m_run + log2f(l_tot)) * kLn2 : -INFINITY;
+  }
+}
+
 // Wide head dims (d = 128 NW, e.g. 512): a 32-key sub-tile of K and V^T is 64 KB at d = 512, so
 // an LDS ring of them would leave one workgroup per CU. Here the head dim is split across the NW
 // waves of a workgroup instead -- wave w owns dims [128 w, 128 w + 128) of one 32-row query group
@@ -1360,6 +1618,19 @@ inline int64_t set_rows(AttnParams& p, int64_t rows) {
   p.group = p.G * p.qsub;
   p.total = p.nbq * p.B * p.Hkv * p.G * p.qsub;
   return (p.total + 8 * p.group - 1) / (8 * p.group) * (8 * p.group);
+}
+
+// 128-row groups of a call (block 64: two query blocks count as one)
+inline int64_t wide_groups(const AttnParams& p) { return p.nbq * p.block / 64 * p.B * p.Hq / 2; }
+
+template <int DT>
+int launch_wide16(AttnParams& p, hipStream_t stream) {
+  const int nw = p.block == 64 || wide_groups(p) < kWide16Full ? 4 : 8;
+  const int64_t grid = set_rows(p, 16 * nw);
+  SSA_REQUIRE(grid < (1ll << 31), SSA_ERR_UNSUPPORTED, "sparse_attn: grid too large");
+  if (nw == 8) sparse_attn_wide16_kernel<DT, 8><<<(unsigned)grid, 512, 0, stream>>>(p);
+  else sparse_attn_wide16_kernel<DT, 4><<<(unsigned)grid, 256, 0, stream>>>(p);
+  return launch_status("sparse_attn_wide16_kernel");
 }
 
 template <int DT>
@@ -1618,6 +1889,8 @@ extern "C" int ssa_sparse_attn_fwd(const void* q, const void* k, const void* v, 
   const size_t vt_bytes = ((size_t)B * Hkv * d * p.n_pad * 2u + 255) / 256 * 256;
   const size_t k16b = k16_bytes(dtype, B, Hkv, p.n_pad, d);
   const bool norms = d == 64 && !(flags & SSA_ATTN_EXACT);
+  if (d == 512 && wide_groups(p) >= kWide16Min)  // (reads V as it is: no V^T pass)
+    return dtype == SSA_BF16 ? launch_wide16<SSA_BF16>(p, st) : launch_wide16<SSA_F16>(p, st);
   if (!(flags & SSA_ATTN_PREPARED))
     SSA_TRY(attn_prepare(k, v, dtype, B, Hkv, n, d, block, p.ksb, p.ksh, p.ksn, p.vsb, p.vsh,
                          p.vsn, workspace, (flags & SSA_ATTN_VT_READY) != 0, norms, st));

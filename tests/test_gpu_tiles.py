@@ -48,3 +48,28 @@ def test_fp32_attention_tiles_match_oracle(cuda, hq, hkv, n, block, W):
                                                                        min(n, (c + 1) * block))]
     s = k[0, h // (hq // hkv), js].astype(np.float64) @ q[0, h, n - 1].astype(np.float64) / 8
     assert abs(float(lse[0, h, n - 1]) - np.log(np.exp(s).sum())) < 1e-5
+
+
+# head dim 512: fewer than 96 groups of 128 rows (32-row workgroups), 4-wave groups (also every
+# block of 64), 8-wave groups; lengths that end inside a wave's rows and inside a 32-key sub-tile
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hq,hkv,n,block,W", [(2, 1, 300, 64, 3), (16, 4, 797, 128, 4),
+                                              (32, 32, 261, 64, 5), (24, 8, 1043, 256, 3),
+                                              (48, 8, 400, 384, 2)])
+def test_d512_attention_tiles_match_oracle(cuda, dtype, hq, hkv, n, block, W):
+    """2e-2: the bar of every 16-bit attention test. The layout is the transformers one (heads
+    inside rows), so no stride is the contiguous one."""
+    rng = np.random.default_rng(n)
+    x = [WL.round_to(rng.standard_normal((1, n, h, 512)).astype(np.float32), dtype)
+         for h in (hq, hkv, hkv)]
+    q, k, v = (a.transpose(0, 2, 1, 3) for a in x)
+    nb = -(-n // block)
+    kv_num, kv_idx = random_lists(rng, hq, nb, min(W, nb))
+    qt, kt, vt = (WL.to_device(a, dtype, cuda).transpose(1, 2) for a in x)
+    out, lse = K.sparse_attention(qt, kt, vt, torch.from_numpy(kv_num).to(cuda),
+                                  torch.from_numpy(kv_idx).to(cuda), block, return_lse=True)
+    heads = [0, hq // 2, hq - 1]
+    ref = O.sparse_attention(q, k, v, kv_num, kv_idx, block, heads=heads)
+    assert np.abs(np_of(out)[:, heads] - ref[:, heads]).max() < 2e-2
+    none = ~np.isfinite(ref[0, 0]).all(-1) | (ref[0, 0] == 0).all(-1)
+    assert (torch.isneginf(lse[0, 0]).cpu().numpy() == none).all()
