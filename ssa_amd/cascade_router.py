@@ -32,6 +32,9 @@ from .ssa_kernel import BLOCK, sparse_attention
 NEG = float("-inf")
 MAX_SEARCH = 1024   # search_k (staged, and committed after escalation) the route kernel takes
 MAX_QUOTA = 2048    # outliers kept per appended chunk
+# Largest block of scores route() has computed ahead of the search, 2 % of an MI355X's HBM (1024
+# query blocks against 20,000 rows take 80 MB); beyond it the search computes them row by row.
+SCORE_WORKSPACE_LIMIT = 6 << 30
 
 
 def _rows(x: torch.Tensor) -> torch.Tensor:
@@ -311,7 +314,7 @@ class CausalCascade:
         rounds = torch.zeros(nbq, dtype=torch.int32, device=dev)
         ix = self.index
         means = self.means
-        ws = None
+        carry = 0
         if ix is not None and certify and self.max_escalations > 0:
             # escalation carry: per query block the best keys of the lists probed so far, as many
             # as the last round's search_k
@@ -319,7 +322,12 @@ class CausalCascade:
             for _ in range(self.max_escalations):
                 sk = min(2 * sk, self.committed)
             skmax = max(min(sk0, self.committed), sk)
-            ws = torch.empty(nbq * skmax, dtype=torch.int64, device=dev)
+            carry = -(-8 * nbq * skmax // 256) * 256
+        # the scores of the staged (and, before the index, the committed) means and the outliers
+        cols = [self.n_sub - self.committed, 0 if ix is not None else self.committed, self.n_out]
+        scores = 4 * nbq * sum(-(-c // 4) * 4 for c in cols)
+        ws_bytes = carry + (scores if scores <= SCORE_WORKSPACE_LIMIT else 0)
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
         _lib.call("ssa_ccc_route", qr.data_ptr(), nbq, qb_start, self.dr,
                   None if means is None else means.data_ptr(), self.committed, self.n_sub,
                   self.spb, None if ix is None else ix.buf.data_ptr(),
@@ -330,7 +338,7 @@ class CausalCascade:
                   self.escalate_factor, self.max_escalations, 1 if certify else 0,
                   float(self.cert_margin), kv_num.data_ptr(), kv_idx.data_ptr(), W,
                   cert.data_ptr(), rounds.data_ptr(), None if ws is None else ws.data_ptr(),
-                  0 if ws is None else 8 * ws.numel(), _lib.stream_of(qr))
+                  ws_bytes, _lib.stream_of(qr))
         stats = {"nbq": nbq, "rounds": rounds,
                  "cert_rate": float(cert.float().mean()) if certify and nbq else None}
         return kv_num, kv_idx, (cert.bool() if certify else None), stats

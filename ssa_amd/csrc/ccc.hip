@@ -97,6 +97,8 @@ __device__ inline float block_max_f32(float x, float* slot) {
   return r;
 }
 
+constexpr int kStreamRun = 4 * kIvfCap;  // candidates of a run once a threshold stands
+
 // Streams M candidates through buf (LDS, kIvfCap keys), keeping the K largest (K <= kIvfMaxSearch,
 // keys unique); keyof(m) is candidate m's key, or 0 to skip it. Once K keys are kept, a candidate
 // below the threshold that kept them (K keys above it already) cannot enter the K largest and is
@@ -110,24 +112,54 @@ __device__ int stream_top(unsigned long long* buf, int64_t M, int K, F keyof, un
   unsigned long long floor_key = 1ull;  // every real key is at least 1
   for (int64_t m0 = 0; m0 < M;) {
     const int room = kIvfCap - nk;
-    const int batch = (int)(M - m0 < room ? M - m0 : room);
-    for (int e = threadIdx.x; e < batch; e += 512) {  // two candidates per thread per pass
-      const bool two = e + 256 < batch;
-      const unsigned long long k0 = keyof(m0 + e);
-      const unsigned long long k1 = two ? keyof(m0 + e + 256) : 0ull;
-      buf[nk + e] = k0 >= floor_key ? k0 : 0ull;
-      if (two) buf[nk + e + 256] = k1 >= floor_key ? k1 : 0ull;
+    int64_t batch = M - m0;
+    bool done = false;
+    if (floor_key > 1ull && batch > room) {
+      // few candidates pass the threshold of the earlier ones: a longer run of them, the keys that
+      // pass appended (if they turn out to be more than the buffer holds, the run is cut as below)
+      if (batch > kStreamRun) batch = kStreamRun;
+      if (threadIdx.x == 0) ws[0] = 0;
+      __syncthreads();
+      for (int e = threadIdx.x; e < batch; e += 512) {
+        const bool two = e + 256 < batch;
+        const unsigned long long k0 = keyof(m0 + e);
+        const unsigned long long k1 = two ? keyof(m0 + e + 256) : 0ull;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const unsigned long long k = u ? k1 : k0;
+          if (k >= floor_key) {
+            const int at = atomicAdd(&ws[0], 1);
+            if (at < room) buf[nk + at] = k;
+          }
+        }
+      }
+      __syncthreads();
+      const int got = ws[0];
+      __syncthreads();  // every thread has read the count before ws is used again
+      if (got <= room) {
+        nk += got;
+        done = true;
+      }
     }
-    __syncthreads();
-    int tot = block_compact<unsigned long long>(buf, nk + batch, buf, ws,
-                                                [](unsigned long long k) { return k != 0ull; });
-    if (tot > K) {
-      const unsigned long long T = block_kth_largest(buf, tot, K, hist, shv);
-      tot = block_compact<unsigned long long>(buf, tot, buf, ws,
-                                              [T](unsigned long long k) { return k >= T; });
+    if (!done) {
+      batch = M - m0 < room ? M - m0 : room;
+      for (int e = threadIdx.x; e < batch; e += 512) {  // two candidates per thread per pass
+        const bool two = e + 256 < batch;
+        const unsigned long long k0 = keyof(m0 + e);
+        const unsigned long long k1 = two ? keyof(m0 + e + 256) : 0ull;
+        buf[nk + e] = k0 >= floor_key ? k0 : 0ull;
+        if (two) buf[nk + e + 256] = k1 >= floor_key ? k1 : 0ull;
+      }
+      __syncthreads();
+      nk = block_compact<unsigned long long>(buf, nk + (int)batch, buf, ws,
+                                             [](unsigned long long k) { return k != 0ull; });
+    }
+    if (nk > K) {
+      const unsigned long long T = block_kth_largest(buf, nk, K, hist, shv);
+      nk = block_compact<unsigned long long>(buf, nk, buf, ws,
+                                             [T](unsigned long long k) { return k >= T; });
       floor_key = T;
     }
-    nk = tot;
     m0 += batch;
   }
   return nk;
@@ -536,6 +568,97 @@ struct CccRouteArgs {
   int32_t* rounds;
   unsigned long long* carry;  // (nbq, kkeep) keys, or NULL: see ccc_route_kernel
   int64_t kkeep;
+  const float* score;  // (nbq, sld) precomputed scores (SCORED), or NULL: see ccc_score_kernel
+  int64_t sld, soff_com, soff_out;  // their row pitch; where the committed / outlier scores start
+  int nstage, nunion;  // the most staged keys and the longest block union of a query block
+};
+
+// Scores of a chunk's query blocks against `m` rows of x (row j0 + c is sub-mean j0 + c of block
+// (j0 + c) / spb; causal: a score is written only if some query block of its tile is past that
+// block): out[q * ld + c] = fl32(<qr_q, x_c>), the fp64 chain in dimension order of dot_row, so
+// the same bits. 64 query blocks x 128 rows per workgroup, both staged in LDS 32 dimensions at a
+// time; a thread owns 4 x 8 chains.
+// In the route kernel a thread read a candidate's row by itself, 64 rows a load instruction: the
+// cache looked up 64 lines per instruction and one workgroup per query block read every row again
+// (3.7 GB for 1024 query blocks x 14,336 rows, 7.7 TB/s). Here a row is read once per 64 query
+// blocks. Measured over a 1M-token
+// prefill (8 chunks of 1024 query blocks, 181 cells): route kernels 2960 us before; 1463 us and 335
+// us of scoring (fp64 fma rate: 25 us for 1024 x 12,288 x 64) with the scores read from memory.
+constexpr int kScoreQ = 64, kScoreC = 128, kScoreD = 32;
+__global__ __launch_bounds__(256) void ccc_score_kernel(const float* __restrict__ qr, int64_t nbq,
+                                                        const float* __restrict__ x, int64_t m,
+                                                        int64_t d, int64_t j0, int64_t spb,
+                                                        int64_t qb_start, int causal,
+                                                        float* __restrict__ out, int64_t ld) {
+  __shared__ __align__(16) float qt[kScoreD][kScoreQ + 4];
+  __shared__ __align__(16) float ct[kScoreD][kScoreC + 4];
+  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
+  const int64_t c0 = (int64_t)blockIdx.x * kScoreC, q0 = (int64_t)blockIdx.y * kScoreQ;
+  const int64_t qlast = q0 + kScoreQ < nbq ? q0 + kScoreQ - 1 : nbq - 1;
+  if (causal && (j0 + c0) / spb >= qb_start + qlast) return;
+  double acc[4][8];
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
+#pragma unroll
+    for (int b = 0; b < 8; ++b) acc[a][b] = 0.0;
+  for (int64_t t0 = 0; t0 < d; t0 += kScoreD) {
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {  // 8 16-byte pieces a row; rows past the end re-read the last
+      const int e = tid + 256 * u, r = e >> 3, p = (e & 7) * 4;
+      const int64_t q = q0 + r < nbq ? q0 + r : nbq - 1;
+      const float4 v = *reinterpret_cast<const float4*>(qr + q * d + t0 + p);
+      qt[p][r] = v.x; qt[p + 1][r] = v.y; qt[p + 2][r] = v.z; qt[p + 3][r] = v.w;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int e = tid + 256 * u, r = e >> 3, p = (e & 7) * 4;
+      const int64_t c = c0 + r < m ? c0 + r : m - 1;
+      const float4 v = *reinterpret_cast<const float4*>(x + c * d + t0 + p);
+      ct[p][r] = v.x; ct[p + 1][r] = v.y; ct[p + 2][r] = v.z; ct[p + 3][r] = v.w;
+    }
+    __syncthreads();
+#pragma unroll 4
+    for (int t = 0; t < kScoreD; ++t) {
+      const float4 q4 = *reinterpret_cast<const float4*>(&qt[t][4 * ty]);
+      const float4 ca = *reinterpret_cast<const float4*>(&ct[t][4 * tx]);
+      const float4 cb = *reinterpret_cast<const float4*>(&ct[t][64 + 4 * tx]);
+      const double qd[4] = {q4.x, q4.y, q4.z, q4.w};
+      const double cd[8] = {ca.x, ca.y, ca.z, ca.w, cb.x, cb.y, cb.z, cb.w};
+#pragma unroll
+      for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int b = 0; b < 8; ++b) acc[a][b] = fma(qd[a], cd[b], acc[a][b]);
+    }
+  }
+  // (ld is a multiple of 4 that holds the columns past m of the last tile's 16-byte stores)
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    const int64_t q = q0 + 4 * ty + a;
+    if (q >= nbq) continue;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int64_t c = c0 + 64 * h + 4 * tx;
+      if (c >= m) continue;
+      const float4 v = {(float)acc[a][4 * h], (float)acc[a][4 * h + 1], (float)acc[a][4 * h + 2],
+                        (float)acc[a][4 * h + 3]};
+      *reinterpret_cast<float4*>(out + q * ld + c) = v;
+    }
+  }
+}
+
+// Sizes of ccc_route_kernel's dynamic LDS arrays: a workgroup's latency is a chain of scans and
+// radix passes with a barrier each, so what matters is how many workgroups a CU holds. With every
+// array at its largest (52 KB, 3 workgroups a CU) a chunk of 1024 query blocks took a second,
+// third-full wave of workgroups; sized by the call it is 22 KB at 181 cells and search_k 32.
+struct CccRouteLds {
+  int staged, cells, list;
+  __host__ __device__ explicit CccRouteLds(const CccRouteArgs& a) {
+    staged = a.nstage;
+    cells = a.has_index ? (int)a.nlist : 0;
+    list = (a.nunion > cells ? a.nunion : cells) + 1;
+  }
+  size_t bytes() const { return (size_t)staged * 8 + (size_t)cells * 4 + (size_t)list * 8; }
 };
 
 // One workgroup per query block i of the chunk (global block qblk = qb_start + i).
@@ -545,13 +668,19 @@ struct CccRouteArgs {
 // through stream_top seeded with them: the top search_k of (the kkeep best of the earlier lists)
 // and (the new lists) is the top search_k of all of them. Each thread reads back only the carry
 // entries it wrote. Without a carry every round scans all of its lists.
-__global__ __launch_bounds__(256) void ccc_route_kernel(CccRouteArgs a) {
+// SCORED: the scores against the staged means, the flat committed means and the outlier keys were
+// written by ccc_score_kernel; the members of probed lists are always scored here.
+template <bool SCORED>
+__global__ __launch_bounds__(256, 4) void ccc_route_kernel(CccRouteArgs a) {
   __shared__ unsigned long long buf[kIvfCap];     // streamed keys, then the merged candidates
-  __shared__ unsigned long long stg[kIvfMaxSearch];  // the staged top
-  __shared__ int lst[kIvfCap];                    // probed lists, then the block union
-  __shared__ int aux[kIvfCap + 1];                // member prefix of the probed lists, then sorted
   __shared__ __align__(16) float qs[kIvfMaxD];
-  __shared__ float csv[kIvfCap];                  // <q, centroid> of every cell
+  // the rest by this call's sizes (CccRouteLds)
+  extern __shared__ unsigned long long dyn[];
+  const CccRouteLds lay(a);
+  unsigned long long* stg = dyn;                              // the staged top
+  float* csv = reinterpret_cast<float*>(dyn + lay.staged);    // <q, centroid> of every cell
+  int* lst = reinterpret_cast<int*>(csv + lay.cells);         // probed lists, then the block union
+  int* aux = lst + lay.list;  // member prefix of the probed lists, then the union sorted
   __shared__ unsigned int hist[256];
   __shared__ unsigned int shv[3];
   __shared__ int ws[4];
@@ -575,6 +704,7 @@ __global__ __launch_bounds__(256) void ccc_route_kernel(CccRouteArgs a) {
   }
   const float* means = a.means;
   const int64_t spb = a.spb, committed = a.committed;
+  const float* score = SCORED ? a.score + i * a.sld : nullptr;
 
   // the staged sub-means (exhaustive, causally masked: parent strictly before the query block)
   const int64_t ns = a.n_sub - committed;
@@ -586,7 +716,7 @@ __global__ __launch_bounds__(256) void ccc_route_kernel(CccRouteArgs a) {
         [&](int64_t m) -> unsigned long long {
           const int64_t j = committed + m;
           if (j / spb >= qblk) return 0ull;
-          return ivf_key(dot_row(qs, means + j * d, d), j);
+          return ivf_key(SCORED ? score[m] : dot_row(qs, means + j * d, d), j);
         },
         hist, shv, ws);
     for (int e = tid; e < nst; e += 256) stg[e] = buf[e];
@@ -614,7 +744,7 @@ __global__ __launch_bounds__(256) void ccc_route_kernel(CccRouteArgs a) {
         ncm = stream_top(
             buf, committed, (int)kc,
             [&](int64_t m) -> unsigned long long {
-              return ivf_key(dot_row(qs, means + m * d, d), m);
+              return ivf_key(SCORED ? score[a.soff_com + m] : dot_row(qs, means + m * d, d), m);
             },
             hist, shv, ws);
       } else {
@@ -741,7 +871,7 @@ __global__ __launch_bounds__(256) void ccc_route_kernel(CccRouteArgs a) {
           buf, a.n_out, cap,
           [&](int64_t r) -> unsigned long long {
             if (op[r] >= qblk) return 0ull;
-            const float s = dot_row(qs, ov + r * d, d);
+            const float s = SCORED ? score[a.soff_out + r] : dot_row(qs, ov + r * d, d);
             return s > tau ? ivf_key(s, r) : 0ull;
           },
           hist, shv, ws);
@@ -1116,6 +1246,8 @@ extern "C" int ssa_ccc_route(const float* qr, int64_t nbq, int64_t qb_start, int
   a.local = local;
   a.ocap = outlier_cap;
   a.ks = search_k_staged;
+  a.nstage = (int)ks;
+  a.nunion = (int)(keep + ocap + win);
   a.sk0 = search_k;
   a.nprobe0 = index != nullptr ? (nprobe < nlist ? nprobe : nlist) : nprobe;
   a.esc = escalate_factor;
@@ -1127,6 +1259,7 @@ extern "C" int ssa_ccc_route(const float* qr, int64_t nbq, int64_t qb_start, int
   a.W = W;
   a.cert = cert;
   a.rounds = rounds;
+  size_t carry_bytes = 0;
   if (index != nullptr && certify && max_escalations > 0) {
     // the escalation carry: nbq rows of skmax keys (skmax >= every round's search_k)
     const size_t need = size_t(nbq) * size_t(skmax) * 8;
@@ -1136,7 +1269,36 @@ extern "C" int ssa_ccc_route(const float* qr, int64_t nbq, int64_t qb_start, int
                 "ccc_route: workspace holds %zu bytes, escalation needs %zu", ws_bytes, need);
     a.carry = static_cast<unsigned long long*>(ws);
     a.kkeep = skmax;
+    carry_bytes = need;
   }
-  ssa::ccc_route_kernel<<<(unsigned)nbq, 256, 0, static_cast<hipStream_t>(stream)>>>(a);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const size_t lds = ssa::CccRouteLds(a).bytes();
+  // precomputed scores, where the workspace has room for them after the carry
+  const int64_t nsr = ks > 0 ? (ns + 3) & ~int64_t(3) : 0;
+  const int64_t ncr = index == nullptr ? (committed + 3) & ~int64_t(3) : 0;
+  const int64_t nor = ocap > 0 ? (n_out + 3) & ~int64_t(3) : 0;
+  const size_t at = (carry_bytes + 255) & ~size_t(255);
+  const size_t sbytes = size_t(nbq) * size_t(nsr + ncr + nor) * 4;
+  const int64_t qtiles = (nbq + ssa::kScoreQ - 1) / ssa::kScoreQ;
+  if (sbytes == 0 || ws == nullptr || ws_bytes < at + sbytes || qtiles > 65535 ||
+      (reinterpret_cast<uintptr_t>(ws) & 15u) != 0) {
+    ssa::ccc_route_kernel<false><<<(unsigned)nbq, 256, lds, st>>>(a);
+    return ssa::launch_status("ccc_route_kernel");
+  }
+  float* sc = reinterpret_cast<float*>(static_cast<char*>(ws) + at);
+  a.score = sc;
+  a.sld = nsr + ncr + nor;
+  a.soff_com = nsr;
+  a.soff_out = nsr + ncr;
+  const auto score = [&](const float* x, int64_t m, int64_t j0, int causal, float* out) {
+    const dim3 g((unsigned)((m + ssa::kScoreC - 1) / ssa::kScoreC), (unsigned)qtiles);
+    ssa::ccc_score_kernel<<<g, 256, 0, st>>>(qr, nbq, x, m, d, j0, spb, qb_start, causal, out,
+                                             a.sld);
+    return ssa::launch_status("ccc_score_kernel");
+  };
+  if (nsr > 0) SSA_TRY(score(means + committed * d, ns, committed, 1, sc));
+  if (ncr > 0) SSA_TRY(score(means, committed, 0, 0, sc + a.soff_com));
+  if (nor > 0) SSA_TRY(score(out_vec, n_out, 0, 0, sc + a.soff_out));
+  ssa::ccc_route_kernel<true><<<(unsigned)nbq, 256, lds, st>>>(a);
   return ssa::launch_status("ccc_route_kernel");
 }

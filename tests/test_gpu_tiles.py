@@ -73,3 +73,33 @@ def test_d512_attention_tiles_match_oracle(cuda, dtype, hq, hkv, n, block, W):
     assert np.abs(np_of(out)[:, heads] - ref[:, heads]).max() < 2e-2
     none = ~np.isfinite(ref[0, 0]).all(-1) | (ref[0, 0] == 0).all(-1)
     assert (torch.isneginf(lse[0, 0]).cpu().numpy() == none).all()
+
+
+# cascade route: query blocks and rows that fill no 64 x 128 score tile, and candidates in rising
+# score order (every run of the streaming search passes the threshold it set, so the run is cut);
+# scored ahead and row by row (no room for the scores)
+@pytest.mark.parametrize("limit", [None, 0])
+@pytest.mark.parametrize("rising", [False, True])
+@pytest.mark.parametrize("d,blocks,nbq", [(64, 2700, 70), (96, 700, 1), (32, 130, 129)])
+def test_cascade_route_scores_match_oracle(cuda, monkeypatch, d, blocks, nbq, rising, limit):
+    from ssa_amd import cascade_router as C
+    if limit is not None:
+        monkeypatch.setattr(C, "SCORE_WORKSPACE_LIMIT", limit)
+    rng = np.random.default_rng(d)
+    n, past = blocks * 128, (blocks - nbq) * 128
+    if rising:
+        k = np.ones((n, d)) * np.repeat(np.arange(n // 32) + 1.0, 32)[:, None] / 1024
+        q = np.ones((nbq * 128, d))
+    else:
+        k, q = rng.standard_normal((n, d)), rng.standard_normal((nbq * 128, d))
+    k, q = (x.astype(np.float16) for x in (k, q))
+    got, ref = C.CausalCascade(d, search_k=48), O.CascadeOracle(d, search_k=48)
+    got.build_threshold = ref.build_threshold = 1 << 30  # every committed mean is scanned
+    for a, b in ((0, past // 2), (past // 2, past), (past, n)):
+        got.append(torch.from_numpy(k[a:b]).to(cuda))
+        ref.append(k[a:b].astype(np.float32))
+    kn, ki, cert, _ = got.route(torch.from_numpy(q).to(cuda), past, certify=True)
+    rn, rl, rc, _ = ref.route(q.astype(np.float32), past, certify=True)
+    assert (kn.cpu().numpy() == rn).all() and (cert.cpu().numpy() == rc).all()
+    for i in range(nbq):
+        assert ki[i, :rn[i]].tolist() == rl[i], i
