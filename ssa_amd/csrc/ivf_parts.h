@@ -206,6 +206,37 @@ __global__ __launch_bounds__(kScoreTile) void ivf_score_kernel(
     if (live[h]) pbest[(bh * gridDim.z + g) * nb + j[h]] = best[h];
 }
 
+// The rank of this thread's centroid a (-1: none) among the threads before it of a 256-thread tile
+// that hold the same one, and trow[c] = how many hold centroid c, for c < nlist <= kIvfCap. A wave
+// finds the lanes that share a centroid with one ballot per bit; their counts (at most 64) meet in
+// wcnt, a byte per (wave, centroid). Walking the tile's 256 centroids in every thread instead took
+// 16-20 us at any size (8192 means, 90
+// centroids: 20.6 -> 4.7 us for the kernel; 4096 means, 181 centroids 16.2 -> 4.2).
+__device__ inline int tile_rank(int a, int64_t nlist, int32_t* __restrict__ trow,
+                                unsigned char (*wcnt)[kIvfCap]) {
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int n16 = (int)((nlist + 15) / 16);
+  for (int e = tid; e < 4 * n16; e += kTile)
+    *reinterpret_cast<u32x4*>(&wcnt[e / n16][16 * (e % n16)]) = u32x4{0u, 0u, 0u, 0u};
+  unsigned long long same = __ballot(a >= 0);
+  for (int b = 0; (1 << b) < nlist; ++b) {
+    const bool one = (a >> b) & 1;
+    const unsigned long long v = __ballot(one);
+    same &= one ? v : ~v;
+  }
+  const int before = __popcll(same & ((1ull << lane) - 1));
+  __syncthreads();  // the counts are zero
+  if (a >= 0 && before == 0) wcnt[w][a] = (unsigned char)__popcll(same);
+  __syncthreads();
+  for (int64_t c = tid; c < nlist; c += kTile)
+    trow[c] = wcnt[0][c] + wcnt[1][c] + wcnt[2][c] + wcnt[3][c];
+  int r = before;
+  if (a >= 0)
+#pragma unroll
+    for (int u = 0; u < 3; ++u) r += u < w ? wcnt[u][a] : 0;
+  return r;
+}
+
 // One workgroup per tile: each block mean joins the best of its groups' centroids; rank = its
 // position among the tile's members of that centroid, and the tile's member count of every
 // centroid goes to its tcount row (0 for absent ones).
@@ -213,13 +244,10 @@ __global__ __launch_bounds__(256) void ivf_rank_kernel(
     const unsigned long long* __restrict__ pbest, int64_t nb, int64_t nlist, int64_t ntiles,
     int64_t groups, int32_t* __restrict__ assign, int32_t* __restrict__ rank,
     int32_t* __restrict__ tcount) {
-  __shared__ int sa[kTile];
-  const int tid = threadIdx.x;
+  __shared__ __align__(16) unsigned char wcnt[4][kIvfCap];
   const int64_t bh = blockIdx.y, tile = blockIdx.x;
-  const int64_t j = tile * kTile + tid;
+  const int64_t j = tile * kTile + threadIdx.x;
   const bool live = j < nb;
-  int32_t* trow = tcount + (bh * ntiles + tile) * nlist;
-  for (int64_t c = tid; c < nlist; c += kTile) trow[c] = 0;
   unsigned long long best = 0ull;
   const unsigned long long* pb = pbest + bh * groups * nb + (live ? j : 0);
   for (int64_t g0 = 0; g0 < groups; g0 += 8) {  // 8 loads in flight (clamped to a valid group)
@@ -230,19 +258,10 @@ __global__ __launch_bounds__(256) void ivf_rank_kernel(
     for (int u = 0; u < 8; ++u) best = k[u] > best ? k[u] : best;
   }
   const int a = live ? (int)ivf_key_index(best) : -1;
-  sa[tid] = a;
-  __syncthreads();  // also orders the zeroing of trow before the counts below
+  const int r = tile_rank(a, nlist, tcount + (bh * ntiles + tile) * nlist, wcnt);
   if (live) {
-    int r = 0;
-    bool last = true;
-    for (int t = 0; t < kTile; ++t) {
-      const int x = sa[t];
-      if (t < tid) r += (x == a);
-      else if (t > tid && x == a) last = false;
-    }
     assign[bh * nb + j] = a;
     rank[bh * nb + j] = r;
-    if (last) trow[a] = r + 1;
   }
 }
 

@@ -103,3 +103,19 @@ def test_cascade_route_scores_match_oracle(cuda, monkeypatch, d, blocks, nbq, ri
     assert (kn.cpu().numpy() == rn).all() and (cert.cpu().numpy() == rc).all()
     for i in range(nbq):
         assert ki[i, :rn[i]].tolist() == rl[i], i
+
+
+# list building: one wave, one tile and several, with remainders; one list, a list per mean, the most
+@pytest.mark.parametrize("nb,nlist", [(33, 1), (64, 64), (256, 17), (257, 257), (1000, 300),
+                                      (2300, 2048)])
+def test_ivf_lists_match_oracle(cuda, nb, nlist):
+    from ssa_amd import ivf_kernel as I
+    rng = np.random.default_rng(nb)
+    mu = rng.standard_normal((2, nb, 32)).astype(np.float32)
+    ix = I.build_ivf(torch.from_numpy(mu).to(cuda), nlist=nlist, niter=1)
+    off, ids = ix.list_offsets.cpu().numpy(), ix.list_ids.cpu().numpy()
+    for h in range(2):
+        cent, lists = O.ivf_build(mu[h], nlist, 1)
+        assert (ix.centroids[h].cpu().numpy() == cent).all()
+        for c in range(nlist):
+            assert ids[h, off[h, c]:off[h, c + 1]].tolist() == lists[c].tolist(), (h, c)
