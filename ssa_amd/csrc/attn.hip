@@ -304,15 +304,6 @@ __global__ __launch_bounds__(256) void transpose_v_kernel(const char* __restrict
   }
 }
 
-// Workgroup barrier once this wave's LDS DMA (global_load_lds) has landed. __syncthreads() is not
-// enough: its workgroup-scope release fence waits for LDS and store traffic (lgkmcnt) only, not
-// for the loads that write LDS asynchronously (vmcnt) -- the compiler's own tracking of them
-// inserted the vmcnt(0) in some builds of the tile loop and not in others. The "memory" clobber
-// keeps the compiler from moving LDS or global accesses across it.
-__device__ inline void dma_barrier() {
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
 // Max / sum of a value with its partner lane (lane ^ 32) without an LDS round trip:
 // permlane32_swap(x, x) returns {x of lanes 0-31 (both halves), x of lanes 32-63 (both halves)}.
 __device__ inline float pair_max(float x) {
@@ -1196,15 +1187,6 @@ struct Mfma16<SSA_F16> {
 
 __device__ inline int kswz(int r) { return (r & 3) | ((r >> 1) & 12); }
 __device__ inline int vswz(int r) { return (r & 3) | ((r >> 1) & 4); }
-
-// Transposing LDS read (ds_read_b64_tr_b16): of the 16 lanes of a group, lane l gives the address
-// of four 16-bit values (its 8 bytes) and receives value l & 3 of lanes 4 j + (l >> 2), j = 0..3:
-// with lane l at row l >> 2, columns 4 (l & 3).. of a 4 x 16 block, column l of the block.
-__device__ inline uint2 lds_read_tr(const unsigned char* p) {
-  typedef short s16x4 __attribute__((ext_vector_type(4)));
-  typedef __attribute__((address_space(3))) s16x4* lds_ptr;
-  return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(p)));
-}
 
 template <int DT, int NW>
 __global__ __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) void sparse_attn_wide16_kernel(AttnParams p) {

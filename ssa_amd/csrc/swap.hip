@@ -72,8 +72,15 @@ __device__ inline f32x16 mfma(float a, float b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
 
-__device__ inline float pair_max(float x) { return fmaxf(x, __shfl_xor(x, 32, 64)); }
-__device__ inline float pair_sum(float x) { return x + __shfl_xor(x, 32, 64); }
+// max / sum of a lane and lane ^ 32 (in lane order, so both get the same bits)
+__device__ inline float pair_max(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ inline float pair_sum(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
 
 // 4 consecutive gradient values of a row: fp32, or rounded to the 16-bit input type DT
 template <int DT>
@@ -181,20 +188,20 @@ __device__ inline unsigned long long bit_range(int lo, int hi) {
 
 // For the key tile [k0, k0 + 64): OR of the tile's block words of one query tile (`any`), and
 // the keys of the tile selected by query-tile row `r` (bit j = key k0 + j; r < 0: none).
-__device__ inline void tile_bits(const unsigned long long* mrow, int64_t k0, int64_t block,
-                                 int64_t nb, int r, unsigned long long& any,
+// (32-bit: at most 8192 blocks of at most 1024 keys.)
+__device__ inline void tile_bits(const unsigned long long* mrow, int64_t k0_, int64_t block_,
+                                 int64_t nb_, int r, unsigned long long& any,
                                  unsigned long long& keys) {
-  const int64_t c0 = k0 / block;
-  int64_t c1 = (k0 + 63) / block;
-  if (c1 > nb - 1) c1 = nb - 1;
+  const int k0 = (int)k0_, block = (int)block_, nb = (int)nb_;
+  const int c0 = (int)((unsigned)k0 / (unsigned)block);
   any = 0ull;
   keys = 0ull;
-  for (int64_t c = c0; c <= c1; ++c) {
+  for (int c = c0; c < nb && c * block <= k0 + 63; ++c) {
     const unsigned long long w = mrow[c];
     any |= w;
     if (r >= 0 && ((w >> r) & 1ull)) {
-      const int64_t a = c * block - k0, e = (c + 1) * block - k0;
-      keys |= bit_range(a < 0 ? 0 : (int)a, e > 64 ? 64 : (int)e);
+      const int a = c * block - k0, e = a + block;
+      keys |= bit_range(a < 0 ? 0 : a, e > 64 ? 64 : e);
     }
   }
 }
@@ -602,14 +609,11 @@ __global__ __launch_bounds__(256, 2) void swap_dkdv_kernel(SwapArgs a) {
 }
 
 // ---- 16-bit inputs: v_mfma_f32_32x32x16_{bf16,f16} ------------------------------------------
-// Tiles stay 16-bit in LDS (row-major stride kRS16, transposed stride kTS16 halves); P and dS are
+// Tiles stay 16-bit in LDS, one copy read along rows and, transposed, along columns; P and dS are
 // rounded to the input type for the second products, as flash attention does. Operand layout
 // (32x32x16): lane l supplies A[l%32][8*(l/32) + j] and B[8*(l/32) + j][l%32], j = 0..7.
 // Head-dim steps t = 0..3 use d = 32*(l/32) + 8t + j; key (query) steps u = 0..1 over a wave's
 // 32 accumulator rows use the rows its registers e = 8u + j hold: 16u + 8*(j/4) + 4*(l/32) + j%4.
-
-constexpr int kRS16 = 72;  // 144 B rows: conflict-free 16-byte reads
-constexpr int kTS16 = 68;  // 136 B rows: conflict-free 8-byte reads
 
 template <int DT>
 struct Mma16;
@@ -641,30 +645,111 @@ __device__ inline u32x4 pack8(const float* x) {
   return r;
 }
 
-// Stages rows [r0, r0 + 64) of a 16-bit (rows, 64) matrix without conversion (256 threads).
-__device__ inline void stage16(const char* base, int64_t rs, int64_t r0, int64_t nrows,
-                               unsigned short* dst, unsigned short* dstT, int tid) {
+// Two 64 x 64 tiles side by side, 8 KB each, go from memory to LDS directly (global_load_lds)
+// while the previous pair is multiplied. 16-byte chunk c of row r sits at chunk c ^ pair_swz(r):
+// the 16 rows of a ds_read_b128 phase and the 4 rows x 64 bytes of a transposing read's phase both
+// hit every bank once, so one copy of a tile serves the product along its rows and the one along
+// its columns.
+// What bounds these kernels is a workgroup's chain of tiles (16 at n 1024: memory latency, products,
+// exponentials, products), not the matrix rate: tiles are loaded one ahead, masks before them, and
+// there are no transposed copies. B 4, 12 heads, n 1024, block 64, top_c 4 + local 2, bf16:
+// forward 47 -> 25 us, dq 50 -> 29, dk / dv 53 -> 38 against tiles staged through registers
+// between two barriers.
+constexpr int kPairTile = 64 * 128;
+__device__ inline int pair_swz(int r) { return ((r & 2) << 1) | ((r >> 2) & 3); }
+
+// Issues this wave's share of rows [r0, r0 + 64) of x and y (row strides in elements; rows past the
+// last one re-read it: their entries are masked) into st and st + kPairTile. 256 threads.
+__device__ inline void issue_pair(const char* x, int64_t xs, const char* y, int64_t ys, int64_t r0,
+                                  int64_t nrows, unsigned char* st, int w, int lane) {
+  const unsigned short* xb = reinterpret_cast<const unsigned short*>(x);
+  const unsigned short* yb = reinterpret_cast<const unsigned short*>(y);
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int c = tid + 256 * i, row = c >> 3, col = (c & 7) * 8;
-    u32x4 w = {0u, 0u, 0u, 0u};
-    if (r0 + row < nrows)
-      w = *reinterpret_cast<const u32x4*>(reinterpret_cast<const unsigned short*>(base) + (r0 + row) * rs + col);
-    if (dst) *reinterpret_cast<u32x4*>(dst + row * kRS16 + col) = w;
-    if (dstT) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        dstT[(col + j) * kTS16 + row] = (unsigned short)((j & 1) ? (w[j >> 1] >> 16) : (w[j >> 1] & 0xffffu));
-    }
+  for (int j = 0; j < 2; ++j) {
+    const int r = (4 * j + w) * 8 + (lane >> 3);
+    const int64_t row = r0 + r < nrows ? r0 + r : nrows - 1;
+    const int col = ((lane & 7) ^ pair_swz(r)) * 8;
+    __builtin_amdgcn_global_load_lds(xb + row * xs + col, st + (4 * j + w) * 1024, 16, 0, 0);
+    __builtin_amdgcn_global_load_lds(yb + row * ys + col, st + kPairTile + (4 * j + w) * 1024, 16,
+                                     0, 0);
   }
 }
 
-__device__ inline u32x4 lds16(const unsigned short* p) { return *reinterpret_cast<const u32x4*>(p); }
-// halves p[0..3] and p[8..11] of a transposed tile row
-__device__ inline u32x4 lds_pair(const unsigned short* p) {
-  typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-  const u32x2 x = *reinterpret_cast<const u32x2*>(p), y = *reinterpret_cast<const u32x2*>(p + 8);
-  return u32x4{x[0], x[1], y[0], y[1]};
+// LDS offsets of a lane's operands in such a tile, for the 32 rows from row 32 * part: `row[t]`
+// the 8 halves of head-dim step t of row 32 part + lo; `col[dh][p]` the transposing reads of the
+// rows 32 part + 8 p + 4 hi .. + 3 at head dim 32 dh + lo (step u: + 2048 u).
+struct PairOffsets {
+  uint32_t row[4], col[2][2];
+  __device__ PairOffsets(int lane, int part) {
+    const int hi = lane >> 5, r = 32 * part + (lane & 31);
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      row[t] = (uint32_t)(r * 128 + (((4 * hi + t) ^ pair_swz(r)) * 16));
+    const int a = lane & 15;
+#pragma unroll
+    for (int dh = 0; dh < 2; ++dh)
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const int k = 32 * part + 8 * p + 4 * hi + (a >> 2);
+        const int c = 4 * dh + 2 * ((lane >> 4) & 1) + ((a & 3) >> 1);
+        col[dh][p] = (uint32_t)(k * 128 + ((c ^ pair_swz(k)) * 16) + (a & 1) * 8);
+      }
+  }
+};
+__device__ inline u32x4 lds16(const unsigned char* p) { return *reinterpret_cast<const u32x4*>(p); }
+__device__ inline u32x4 lds_cols(const unsigned char* st, const PairOffsets& o, int dh, int u) {
+  const uint2 x = lds_read_tr(st + o.col[dh][0] + 2048 * u);
+  const uint2 y = lds_read_tr(st + o.col[dh][1] + 2048 * u);
+  return u32x4{x.x, x.y, y.x, y.y};
+}
+
+// Cursor over the key tiles of a query tile that hold a selected key: lane t tests tile 64 c + t,
+// one round of loads per 64 tiles. The same in every wave of the workgroup.
+struct TileCursor {
+  const unsigned long long* mrow;
+  int block, nb, nkt, chunk;
+  unsigned long long act, word;  // word: this lane's tile's rows (any of its blocks)
+  __device__ int next(int kt, int lane) {
+    while (kt < nkt) {
+      const int c0 = kt & ~63;
+      if (c0 != chunk) {
+        unsigned long long any = 0ull, unused;
+        if (c0 + lane < nkt) tile_bits(mrow, (c0 + lane) * 64, block, nb, -1, any, unused);
+        act = __ballot(any != 0ull);
+        word = any;
+        chunk = c0;
+      }
+      const unsigned long long rest = act & (~0ull << (kt - c0));
+      if (rest != 0ull) return c0 + __builtin_ctzll(rest);
+      kt = c0 + 64;
+    }
+    return nkt;
+  }
+  // the keys of tile kt (the last next()) that row r of the query tile attends, at most key row q
+  // (r < 0: none), as the 32 bits from key `from` on. A tile inside one block (block a multiple of
+  // 64) needs only the word next() loaded, read from its lane: no memory wait per tile.
+  __device__ unsigned int keys(int kt, int r, int q, int from) const {
+    unsigned long long any, k;
+    if (block % 64 == 0) {
+      const unsigned int lo = __builtin_amdgcn_readlane((unsigned int)word, kt - chunk);
+      const unsigned int hi = __builtin_amdgcn_readlane((unsigned int)(word >> 32), kt - chunk);
+      const unsigned int half = r & 32 ? hi : lo;
+      k = r >= 0 && ((half >> (r & 31)) & 1u) ? ~0ull : 0ull;
+    } else {
+      tile_bits(mrow, kt * 64, block, nb, r, any, k);
+    }
+    const int past = q - kt * 64;
+    if (past < 63) k &= past < 0 ? 0ull : (2ull << past) - 1ull;
+    return (unsigned int)(k >> from);
+  }
+};
+
+// All ones if bit c of bits is set, else 0 (one v_bfe_i32); x where it is, else `other` (v_bfi_b32).
+__device__ inline unsigned int bit_mask(unsigned int bits, int c) {
+  return (unsigned int)__builtin_amdgcn_sbfe((int)bits, c, 1);
+}
+__device__ inline float masked(float x, unsigned int mask, float other) {
+  return __uint_as_float((__float_as_uint(x) & mask) | (__float_as_uint(other) & ~mask));
 }
 
 // one row's 32 halves [32*hi, 32*hi + 32) as 4 packed operands (zeros when !valid)
@@ -678,12 +763,10 @@ __device__ inline void load_row16(const char* base, int64_t off, bool valid, u32
 }
 
 template <int DT>
-__global__ __launch_bounds__(256) void swap_fwd16_kernel(SwapArgs a) {
-  // K and V^T tiles (17920 B), later the 34 x 128-float merge buffer (17408 B)
-  __shared__ __attribute__((aligned(16))) char smem[64 * kRS16 * 2 + 64 * kTS16 * 2];
-  static_assert(64 * kRS16 * 2 + 64 * kTS16 * 2 >= 34 * 128 * 4, "merge buffer");
-  unsigned short* ks = reinterpret_cast<unsigned short*>(smem);  // K [key][d]
-  unsigned short* vt = ks + 64 * kRS16;                          // V [d][key]
+__global__ __launch_bounds__(256, 4) void swap_fwd16_kernel(SwapArgs a) {
+  __shared__ __attribute__((aligned(1024))) unsigned char st0[2 * kPairTile];  // K, V tiles
+  __shared__ __attribute__((aligned(1024))) unsigned char st1[2 * kPairTile];
+  __shared__ float ml[2 * 128];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, hi = lane >> 5, lo = lane & 31;
   const int qh = w & 1, kh = w >> 1;
   const int64_t nbh = a.B * a.Hq;
@@ -708,67 +791,85 @@ __global__ __launch_bounds__(256) void swap_fwd16_kernel(SwapArgs a) {
     for (int e = 0; e < 16; ++e) o[x][e] = 0.0f;
   int64_t qlast = q0 + 63;
   if (qlast > a.n - 1) qlast = a.n - 1;
-  const int64_t nkt = qlast / 64 + 1;
-  for (int64_t kt = 0; kt < nkt; ++kt) {
-    const int64_t k0 = kt * 64;
-    unsigned long long any, keys;
-    tile_bits(mrow, k0, a.block, a.nb, qvalid ? r : -1, any, keys);
-    if (any == 0ull) continue;
-    __syncthreads();
-    stage16(kb, a.ksn, k0, a.n, ks, nullptr, tid);
-    stage16(vb, a.vsn, k0, a.n, nullptr, vt, tid);
-    __syncthreads();
+  TileCursor cur{mrow, (int)a.block, (int)a.nb, (int)(qlast / 64) + 1, -1, 0ull, 0ull};
+  const int nkt = cur.nkt;
+  const PairOffsets off(lane, kh);
+  auto key_bits = [&](int kt) {
+    return cur.keys(kt, qvalid ? r : -1, (int)qi, 32 * kh + 4 * hi);
+  };
+  auto compute = [&](const unsigned char* st, unsigned int keys) {
+    if (!__any(keys != 0u)) return;  // no row of the wave attends a key of its half
     f32x16 s;
 #pragma unroll
     for (int e = 0; e < 16; ++e) s[e] = 0.0f;
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
-      s = Mma16<DT>::mma(lds16(ks + (32 * kh + lo) * kRS16 + 32 * hi + 8 * t), qv[t], s);
+    for (int t = 0; t < 4; ++t) s = Mma16<DT>::mma(lds16(st + off.row[t]), qv[t], s);
     float mx = -INFINITY;
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
-      const int kk = 32 * kh + (e >> 2) * 8 + hi * 4 + (e & 3);
-      const bool ok = ((keys >> kk) & 1ull) && (k0 + kk <= qi);
-      s[e] = ok ? s[e] * sl2 : -INFINITY;
+      s[e] = masked(s[e], bit_mask(keys, (e >> 2) * 8 + (e & 3)), -INFINITY);
       mx = fmaxf(mx, s[e]);
     }
-    mx = pair_max(mx);
-    const float mnew = fmaxf(m, mx);
-    const float alpha = mnew == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - mnew);
+    const float mnew = fmaxf(m, pair_max(mx) * sl2);
+    if (__any(mnew > m)) {  // (rare after the first tiles)
+      const float alpha = mnew > m ? __builtin_amdgcn_exp2f(m - mnew) : 1.0f;
+      l *= alpha;
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o[x][e] *= alpha;
+      m = mnew;
+    }
+    const float mref = m == -INFINITY ? 0.0f : m;
     float p[16];
-    float ps = 0.0f;
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
-      p[e] = s[e] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(s[e] - mnew);
-      ps += p[e];
+      p[e] = __builtin_amdgcn_exp2f(fmaf(s[e], sl2, -mref));
+      l += p[e];
     }
-    l = l * alpha + ps;
-    m = mnew;
-#pragma unroll
-    for (int x = 0; x < 2; ++x)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) o[x][e] *= alpha;
     const u32x4 p0 = pack8<DT>(p), p1 = pack8<DT>(p + 8);
 #pragma unroll
     for (int dh = 0; dh < 2; ++dh) {
-      const unsigned short* vrow = vt + (32 * dh + lo) * kTS16 + 32 * kh + 4 * hi;
-      o[dh] = Mma16<DT>::mma(lds_pair(vrow), p0, o[dh]);
-      o[dh] = Mma16<DT>::mma(lds_pair(vrow + 16), p1, o[dh]);
+      o[dh] = Mma16<DT>::mma(lds_cols(st + kPairTile, off, dh, 0), p0, o[dh]);
+      o[dh] = Mma16<DT>::mma(lds_cols(st + kPairTile, off, dh, 1), p1, o[dh]);
     }
+  };
+  int kt = cur.next(0, lane);
+  unsigned int keys = 0u;
+  if (kt < nkt) {
+    keys = key_bits(kt);
+    issue_pair(kb, a.ksn, vb, a.vsn, (int64_t)kt * 64, a.n, st0, w, lane);
+  }
+  while (kt < nkt) {
+    int nxt = cur.next(kt + 1, lane);
+    unsigned int nkeys = nxt < nkt ? key_bits(nxt) : 0u;
+    dma_barrier();  // st0 has landed for every wave; st1 is no longer read
+    if (nxt < nkt) issue_pair(kb, a.ksn, vb, a.vsn, (int64_t)nxt * 64, a.n, st1, w, lane);
+    compute(st0, keys);
+    kt = nxt;
+    if (kt >= nkt) break;
+    keys = nkeys;
+    nxt = cur.next(kt + 1, lane);
+    nkeys = nxt < nkt ? key_bits(nxt) : 0u;
+    dma_barrier();  // st1 has landed; st0 is no longer read
+    if (nxt < nkt) issue_pair(kb, a.ksn, vb, a.vsn, (int64_t)nxt * 64, a.n, st0, w, lane);
+    compute(st1, keys);
+    kt = nxt;
+    keys = nkeys;
   }
   l = pair_sum(l);
   __syncthreads();
-  float* buf = reinterpret_cast<float*>(smem);  // 34 x 128 floats
+  float* buf = reinterpret_cast<float*>(st0);  // 32 x 128 floats
   const int slot = qh * 64 + lane;
   if (kh == 1) {
-    buf[slot] = m;
-    buf[128 + slot] = l;
+    ml[slot] = m;
+    ml[128 + slot] = l;
 #pragma unroll
-    for (int x = 0; x < 32; ++x) buf[(2 + x) * 128 + slot] = o[x >> 4][x & 15];
+    for (int x = 0; x < 32; ++x) buf[x * 128 + slot] = o[x >> 4][x & 15];
   }
   __syncthreads();
   if (kh == 1 || !qvalid) return;
-  const float m1 = buf[slot], l1 = buf[128 + slot];
+  const float m1 = ml[slot], l1 = ml[128 + slot];
   const float M = fmaxf(m, m1);
   const float a0 = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - M);
   const float a1 = m1 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m1 - M);
@@ -776,7 +877,7 @@ __global__ __launch_bounds__(256) void swap_fwd16_kernel(SwapArgs a) {
   const float inv = 1.0f / lt;
   float of[32];
 #pragma unroll
-  for (int x = 0; x < 32; ++x) of[x] = (o[x >> 4][x & 15] * a0 + buf[(2 + x) * 128 + slot] * a1) * inv;
+  for (int x = 0; x < 32; ++x) of[x] = (o[x >> 4][x & 15] * a0 + buf[x * 128 + slot] * a1) * inv;
   const int64_t ooff = b * a.osb + h * a.osh + qi * a.osn;
 #pragma unroll
   for (int dh = 0; dh < 2; ++dh)
@@ -789,12 +890,9 @@ __global__ __launch_bounds__(256) void swap_fwd16_kernel(SwapArgs a) {
 }
 
 template <int DT>
-__global__ __launch_bounds__(256) void swap_dq16_kernel(SwapArgs a) {
-  __shared__ __attribute__((aligned(16))) char smem[2 * 64 * kRS16 * 2 + 64 * kTS16 * 2];
-  static_assert(2 * 64 * kRS16 * 2 + 64 * kTS16 * 2 >= 32 * 128 * 4, "merge buffer");
-  unsigned short* ks = reinterpret_cast<unsigned short*>(smem);  // K [key][d]
-  unsigned short* vs = ks + 64 * kRS16;                          // V [key][d]
-  unsigned short* kt_ = vs + 64 * kRS16;                         // K [d][key]
+__global__ __launch_bounds__(256, 3) void swap_dq16_kernel(SwapArgs a) {
+  __shared__ __attribute__((aligned(1024))) unsigned char st0[2 * kPairTile];  // K, V tiles
+  __shared__ __attribute__((aligned(1024))) unsigned char st1[2 * kPairTile];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, hi = lane >> 5, lo = lane & 31;
   const int qh = w & 1, kh = w >> 1;
   const int64_t nbh = a.B * a.Hq;
@@ -834,16 +932,14 @@ __global__ __launch_bounds__(256) void swap_dq16_kernel(SwapArgs a) {
     for (int e = 0; e < 16; ++e) dqa[x][e] = 0.0f;
   int64_t qlast = q0 + 63;
   if (qlast > a.n - 1) qlast = a.n - 1;
-  const int64_t nkt = qlast / 64 + 1;
-  for (int64_t kt = 0; kt < nkt; ++kt) {
-    const int64_t k0 = kt * 64;
-    unsigned long long any, keys;
-    tile_bits(mrow, k0, a.block, a.nb, qvalid ? r : -1, any, keys);
-    if (any == 0ull) continue;
-    __syncthreads();
-    stage16(kb, a.ksn, k0, a.n, ks, kt_, tid);
-    stage16(vb, a.vsn, k0, a.n, vs, nullptr, tid);
-    __syncthreads();
+  TileCursor cur{mrow, (int)a.block, (int)a.nb, (int)(qlast / 64) + 1, -1, 0ull, 0ull};
+  const int nkt = cur.nkt;
+  const PairOffsets off(lane, kh);
+  auto key_bits = [&](int kt) {
+    return cur.keys(kt, qvalid ? r : -1, (int)qi, 32 * kh + 4 * hi);
+  };
+  auto compute = [&](const unsigned char* st, unsigned int keys) {
+    if (!__any(keys != 0u)) return;  // no row of the wave attends a key of its half
     f32x16 s, dp;
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
@@ -852,28 +948,48 @@ __global__ __launch_bounds__(256) void swap_dq16_kernel(SwapArgs a) {
     }
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      const int off = (32 * kh + lo) * kRS16 + 32 * hi + 8 * t;
-      s = Mma16<DT>::mma(lds16(ks + off), qv[t], s);
-      dp = Mma16<DT>::mma(lds16(vs + off), gv[t], dp);
+      s = Mma16<DT>::mma(lds16(st + off.row[t]), qv[t], s);
+      dp = Mma16<DT>::mma(lds16(st + kPairTile + off.row[t]), gv[t], dp);
     }
     float ds[16];
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
-      const int kk = 32 * kh + (e >> 2) * 8 + hi * 4 + (e & 3);
-      const bool ok = ((keys >> kk) & 1ull) && (k0 + kk <= qi);
-      const float p = ok ? __builtin_amdgcn_exp2f(fmaf(s[e], sl2, -lse2)) : 0.0f;
+      const float p = masked(__builtin_amdgcn_exp2f(fmaf(s[e], sl2, -lse2)),
+                             bit_mask(keys, (e >> 2) * 8 + (e & 3)), 0.0f);
       ds[e] = p * (dp[e] - Di);
     }
     const u32x4 d0 = pack8<DT>(ds), d1 = pack8<DT>(ds + 8);
 #pragma unroll
     for (int dh = 0; dh < 2; ++dh) {
-      const unsigned short* krow = kt_ + (32 * dh + lo) * kTS16 + 32 * kh + 4 * hi;
-      dqa[dh] = Mma16<DT>::mma(lds_pair(krow), d0, dqa[dh]);
-      dqa[dh] = Mma16<DT>::mma(lds_pair(krow + 16), d1, dqa[dh]);
+      dqa[dh] = Mma16<DT>::mma(lds_cols(st, off, dh, 0), d0, dqa[dh]);
+      dqa[dh] = Mma16<DT>::mma(lds_cols(st, off, dh, 1), d1, dqa[dh]);
     }
+  };
+  int kt = cur.next(0, lane);
+  unsigned int keys = 0u;
+  if (kt < nkt) {
+    keys = key_bits(kt);
+    issue_pair(kb, a.ksn, vb, a.vsn, (int64_t)kt * 64, a.n, st0, w, lane);
+  }
+  while (kt < nkt) {
+    int nxt = cur.next(kt + 1, lane);
+    unsigned int nkeys = nxt < nkt ? key_bits(nxt) : 0u;
+    dma_barrier();  // st0 has landed for every wave; st1 is no longer read
+    if (nxt < nkt) issue_pair(kb, a.ksn, vb, a.vsn, (int64_t)nxt * 64, a.n, st1, w, lane);
+    compute(st0, keys);
+    kt = nxt;
+    if (kt >= nkt) break;
+    keys = nkeys;
+    nxt = cur.next(kt + 1, lane);
+    nkeys = nxt < nkt ? key_bits(nxt) : 0u;
+    dma_barrier();  // st1 has landed; st0 is no longer read
+    if (nxt < nkt) issue_pair(kb, a.ksn, vb, a.vsn, (int64_t)nxt * 64, a.n, st0, w, lane);
+    compute(st1, keys);
+    kt = nxt;
+    keys = nkeys;
   }
   __syncthreads();
-  float* buf = reinterpret_cast<float*>(smem);  // 32 x 128 floats
+  float* buf = reinterpret_cast<float*>(st0);  // 32 x 128 floats
   const int slot = qh * 64 + lane;
   if (kh == 1) {
 #pragma unroll
@@ -895,14 +1011,10 @@ __global__ __launch_bounds__(256) void swap_dq16_kernel(SwapArgs a) {
 
 template <int DT>
 __global__ __launch_bounds__(256, 2) void swap_dkdv16_kernel(SwapArgs a) {
-  __shared__ __attribute__((aligned(16))) char smem[2 * 64 * kRS16 * 2 + 2 * 64 * kTS16 * 2];
-  static_assert(2 * 64 * kRS16 * 2 + 2 * 64 * kTS16 * 2 >= 2 * 32 * 128 * 4, "merge buffers");
-  __shared__ float lse_s[64], del_s[64];
+  __shared__ __attribute__((aligned(1024))) unsigned char st0[2 * kPairTile];  // Q, dO tiles
+  __shared__ __attribute__((aligned(1024))) unsigned char st1[2 * kPairTile];
+  __shared__ float ld_s[2][2][64];  // [stage][lse, delta][row]
   __shared__ unsigned long long act_s[4];
-  unsigned short* qs = reinterpret_cast<unsigned short*>(smem);  // Q [q][d]
-  unsigned short* gs = qs + 64 * kRS16;                          // dO [q][d]
-  unsigned short* qtT = gs + 64 * kRS16;                         // Q [d][q]
-  unsigned short* gtT = qtT + 64 * kTS16;                        // dO [d][q]
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, hi = lane >> 5, lo = lane & 31;
   const int kq = w & 1, qp = w >> 1;
   const int64_t nbkv = a.B * a.Hkv;
@@ -925,62 +1037,99 @@ __global__ __launch_bounds__(256, 2) void swap_dkdv16_kernel(SwapArgs a) {
       dka[x][e] = 0.0f;
       dva[x][e] = 0.0f;
     }
-  for (int64_t g = 0; g < a.G; ++g) {
-    const int64_t hq = kvh * a.G + g, bh = b * a.Hq + hq;
-    const char* qb = a.q + (b * a.qsb + hq * a.qsh) * 2;
-    const char* gb = a.dout + (b * a.osb + hq * a.osh) * 2;
-    int64_t chunk = -1;
-    int64_t qt = next_active_tile(a, bh, k0, k0 / 64, act_s, chunk);
-    while (qt < a.nqt) {
-      const int64_t nxt = next_active_tile(a, bh, k0, qt + 1, act_s, chunk);
-      const unsigned long long* mrow = a.masks + (bh * a.nqt + qt) * a.nb;
-      const unsigned long long mw = kvalid ? mrow[ck] : 0ull;
-      const int64_t q0 = qt * 64;
-      __syncthreads();  // the previous tile's compute is done with the LDS tiles
-      stage16(qb, a.qsn, q0, a.n, qs, qtT, tid);
-      stage16(gb, a.osn, q0, a.n, gs, gtT, tid);
-      if (tid < 64) {
-        const bool ok = q0 + tid < a.n;
-        lse_s[tid] = ok ? a.lse[bh * a.n + q0 + tid] * kLog2eS : 0.0f;
-        del_s[tid] = ok ? a.delta[bh * a.n + q0 + tid] : 0.0f;
-      }
-      __syncthreads();
-      f32x16 s, dp;
+  const PairOffsets off(lane, qp);
+  auto compute = [&](const unsigned char* st, const float (*ld)[64], unsigned int rows) {
+    if (!__any(rows != 0u)) return;  // no row of the wave's half attends a key of its half
+    f32x16 s, dp;
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        s[e] = 0.0f;
-        dp[e] = 0.0f;
-      }
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int off = (32 * qp + lo) * kRS16 + 32 * hi + 8 * t;
-        s = Mma16<DT>::mma(lds16(qs + off), kv[t], s);
-        dp = Mma16<DT>::mma(lds16(gs + off), vv[t], dp);
-      }
-      float p[16], ds[16];
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int qq = 32 * qp + (e >> 2) * 8 + hi * 4 + (e & 3);
-        const bool ok = ((mw >> qq) & 1ull) && (key <= q0 + qq);
-        p[e] = ok ? __builtin_amdgcn_exp2f(fmaf(s[e], sl2, -lse_s[qq])) : 0.0f;
-        ds[e] = p[e] * (dp[e] - del_s[qq]);
-      }
-      const u32x4 p0 = pack8<DT>(p), p1 = pack8<DT>(p + 8);
-      const u32x4 d0 = pack8<DT>(ds), d1 = pack8<DT>(ds + 8);
-#pragma unroll
-      for (int dh = 0; dh < 2; ++dh) {
-        const int off = (32 * dh + lo) * kTS16 + 32 * qp + 4 * hi;
-        dva[dh] = Mma16<DT>::mma(lds_pair(gtT + off), p0, dva[dh]);
-        dva[dh] = Mma16<DT>::mma(lds_pair(gtT + off + 16), p1, dva[dh]);
-        dka[dh] = Mma16<DT>::mma(lds_pair(qtT + off), d0, dka[dh]);
-        dka[dh] = Mma16<DT>::mma(lds_pair(qtT + off + 16), d1, dka[dh]);
-      }
-      qt = nxt;
+    for (int e = 0; e < 16; ++e) {
+      s[e] = 0.0f;
+      dp[e] = 0.0f;
     }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      s = Mma16<DT>::mma(lds16(st + off.row[t]), kv[t], s);
+      dp = Mma16<DT>::mma(lds16(st + kPairTile + off.row[t]), vv[t], dp);
+    }
+    float p[16], ds[16];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int qq = 32 * qp + (e >> 2) * 8 + hi * 4 + (e & 3);
+      p[e] = masked(__builtin_amdgcn_exp2f(fmaf(s[e], sl2, -ld[0][qq])),
+                    bit_mask(rows, (e >> 2) * 8 + (e & 3)), 0.0f);
+      ds[e] = p[e] * (dp[e] - ld[1][qq]);
+    }
+    const u32x4 p0 = pack8<DT>(p), p1 = pack8<DT>(p + 8);
+    const u32x4 d0 = pack8<DT>(ds), d1 = pack8<DT>(ds + 8);
+#pragma unroll
+    for (int dh = 0; dh < 2; ++dh) {
+      dva[dh] = Mma16<DT>::mma(lds_cols(st + kPairTile, off, dh, 0), p0, dva[dh]);
+      dva[dh] = Mma16<DT>::mma(lds_cols(st + kPairTile, off, dh, 1), p1, dva[dh]);
+      dka[dh] = Mma16<DT>::mma(lds_cols(st, off, dh, 0), d0, dka[dh]);
+      dka[dh] = Mma16<DT>::mma(lds_cols(st, off, dh, 1), d1, dka[dh]);
+    }
+  };
+  // The walk over (query head, query tile) pairs. A pair's mask word and (threads 0..127) its row's
+  // lse or delta are loaded one pair before its tiles are, two before it is multiplied.
+  struct Pair {
+    int64_t g, qt;
+    unsigned long long mw;
+    float ld;
+  };
+  int64_t chunk = -1;
+  auto next_pair = [&](Pair at) {  // the pair at or after `at`; g == G: none left
+    for (; at.g < a.G; ++at.g, at.qt = k0 / 64, chunk = -1) {
+      const int64_t bh = b * a.Hq + kvh * a.G + at.g;
+      at.qt = next_active_tile(a, bh, k0, at.qt, act_s, chunk);
+      if (at.qt < a.nqt) {
+        at.mw = kvalid ? a.masks[(bh * a.nqt + at.qt) * a.nb + ck] : 0ull;
+        const int64_t row = at.qt * 64 + lane;
+        if (tid < 128)  // (rows past the end belong to no list: any finite value will do)
+          at.ld = (tid < 64 ? a.lse : a.delta)[bh * a.n + (row < a.n ? row : a.n - 1)];
+        break;
+      }
+    }
+    return at;
+  };
+  auto after = [&](Pair at) {
+    if (at.g >= a.G) return at;
+    ++at.qt;
+    return next_pair(at);
+  };
+  auto issue = [&](const Pair& at, unsigned char* st, float (*ld)[64]) {
+    const int64_t hq = kvh * a.G + at.g;
+    issue_pair(a.q + (b * a.qsb + hq * a.qsh) * 2, a.qsn, a.dout + (b * a.osb + hq * a.osh) * 2,
+               a.osn, at.qt * 64, a.n, st, w, lane);
+    if (tid < 128) ld[tid >> 6][lane] = tid < 64 ? at.ld * kLog2eS : at.ld;
+  };
+  // the rows of the lane's half that attend its key, as the 32 bits from row 32 qp + 4 hi on
+  auto rows_of = [&](const Pair& at) {
+    unsigned long long mw = at.mw;
+    const int ahead = (int)(key - at.qt * 64);  // token causal: rows at or after the key
+    if (ahead > 0) mw &= ~0ull << ahead;        // (< 64: the walk starts at the key's tile)
+    return (unsigned int)(mw >> (32 * qp + 4 * hi));
+  };
+  Pair at = next_pair(Pair{0, k0 / 64, 0ull, 0.0f});
+  if (at.g < a.G) issue(at, st0, ld_s[0]);
+  Pair nx = after(at);
+  while (at.g < a.G) {
+    dma_barrier();  // stage 0 has landed for every wave; stage 1 is no longer read
+    if (nx.g < a.G) issue(nx, st1, ld_s[1]);
+    Pair nn = after(nx);
+    compute(st0, ld_s[0], rows_of(at));
+    at = nx;
+    nx = nn;
+    if (at.g >= a.G) break;
+    dma_barrier();  // stage 1 has landed; stage 0 is no longer read
+    if (nx.g < a.G) issue(nx, st0, ld_s[0]);
+    nn = after(nx);
+    compute(st1, ld_s[1], rows_of(at));
+    at = nx;
+    nx = nn;
   }
   __syncthreads();
-  float* bk = reinterpret_cast<float*>(smem);  // 32 x 128 floats each
-  float* bv = bk + 32 * 128;
+  float* bk = reinterpret_cast<float*>(st0);  // 32 x 128 floats each
+  float* bv = reinterpret_cast<float*>(st1);
   const int slot = kq * 64 + lane;
   if (qp == 1) {
 #pragma unroll
