@@ -17,9 +17,8 @@
 //                     and the query tiles at or after the key tile: S = Q K^T, dP = dO V^T,
 //                     dV^T += dO^T P, dK^T += Q^T dS.
 // Workgroups are issued longest first (the last query tiles, the first key tiles).
-// The dq and dk/dv passes each own their outputs (no atomics, deterministic). Inputs of any
-// dtype are staged through LDS as fp32; products and sums are fp32 (the reference trains the
-// swap in fp32).
+// The dq and dk/dv passes each own their outputs (no atomics, deterministic). fp32 inputs:
+// products and sums are fp32 (the reference trains the swap in fp32); 16-bit inputs: below.
 //
 // MFMA operand layout (32x32x2 f32): lane l supplies A[l%32][l/32] and B[l/32][l%32]; the result
 // lane l, register r holds C[(r/4)*8 + (l/32)*4 + r%4][l%32]. The contraction index k of a step
@@ -36,8 +35,6 @@ size_t masked_tiled_workspace(int64_t B, int64_t Hq, int64_t n, int64_t block);
 
 namespace {
 
-constexpr int kLS = 68;                 // LDS row stride (floats): conflict-free 16-byte reads
-constexpr int kTileFloats = 64 * kLS;
 constexpr int kMaxMaskBlocks = 8192;    // key blocks per sequence (LDS of the mask builder)
 constexpr float kLog2eS = 1.4426950408889634f;
 constexpr float kLn2S = 0.6931471805599453f;
@@ -97,45 +94,6 @@ __device__ inline void store_grad4(void* base, int64_t off, const f32x4& v, bool
     *reinterpret_cast<uint2*>(static_cast<unsigned short*>(base) + off) = u;
   } else {
     *reinterpret_cast<f32x4*>(static_cast<float*>(base) + off) = v;
-  }
-}
-
-// Stages rows [r0, r0 + 64) (rows >= nrows read as zeros) of a (rows, 64) matrix with row stride
-// rs elements into LDS as fp32 with 256 threads: row-major into dst and/or transposed into dstT.
-template <int DT>
-__device__ inline void stage_tile(const char* base, int64_t rs, int64_t r0, int64_t nrows,
-                                  float* dst, float* dstT, int tid) {
-  if constexpr (DT == SSA_F32) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int c = tid + 256 * i, row = c >> 4, col = (c & 15) * 4;
-      f32x4 x = {0.0f, 0.0f, 0.0f, 0.0f};
-      if (r0 + row < nrows)
-        x = *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(base) + (r0 + row) * rs + col);
-      if (dst) *reinterpret_cast<f32x4*>(dst + row * kLS + col) = x;
-      if (dstT) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) dstT[(col + j) * kLS + row] = x[j];
-      }
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int c = tid + 256 * i, row = c >> 3, col = (c & 7) * 8;
-      u32x4 w = {0u, 0u, 0u, 0u};
-      if (r0 + row < nrows)
-        w = *reinterpret_cast<const u32x4*>(reinterpret_cast<const unsigned short*>(base) + (r0 + row) * rs + col);
-      float f[8];
-      unpack8(w, f, DT == SSA_BF16);
-      if (dst) {
-        *reinterpret_cast<f32x4*>(dst + row * kLS + col) = f32x4{f[0], f[1], f[2], f[3]};
-        *reinterpret_cast<f32x4*>(dst + row * kLS + col + 4) = f32x4{f[4], f[5], f[6], f[7]};
-      }
-      if (dstT) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) dstT[(col + j) * kLS + row] = f[j];
-      }
-    }
   }
 }
 
@@ -236,10 +194,107 @@ __global__ __launch_bounds__(256) void row_block_masks_kernel(SwapArgs a) {
 // wave contracts over; the two y halves keep separate softmax / gradient state and are merged
 // through LDS at the end. dk/dv: x picks the 32 keys, y the 32 query rows of each query tile.
 
-template <int DT>
+// Cursor over the key tiles of a query tile that hold a selected key: lane t tests tile 64 c + t,
+// one round of loads per 64 tiles. The same in every wave of the workgroup.
+struct TileCursor {
+  const unsigned long long* mrow;
+  int block, nb, nkt, chunk;
+  unsigned long long act, word;  // word: this lane's tile's rows (any of its blocks)
+  __device__ int next(int kt, int lane) {
+    while (kt < nkt) {
+      const int c0 = kt & ~63;
+      if (c0 != chunk) {
+        unsigned long long any = 0ull, unused;
+        if (c0 + lane < nkt) tile_bits(mrow, (c0 + lane) * 64, block, nb, -1, any, unused);
+        act = __ballot(any != 0ull);
+        word = any;
+        chunk = c0;
+      }
+      const unsigned long long rest = act & (~0ull << (kt - c0));
+      if (rest != 0ull) return c0 + __builtin_ctzll(rest);
+      kt = c0 + 64;
+    }
+    return nkt;
+  }
+  // the keys of tile kt (the last next()) that row r of the query tile attends, at most key row q
+  // (r < 0: none), as the 32 bits from key `from` on. A tile inside one block (block a multiple of
+  // 64) needs only the word next() loaded, read from its lane: no memory wait per tile.
+  __device__ unsigned int keys(int kt, int r, int q, int from) const {
+    unsigned long long any, k;
+    if (block % 64 == 0) {
+      const unsigned int lo = __builtin_amdgcn_readlane((unsigned int)word, kt - chunk);
+      const unsigned int hi = __builtin_amdgcn_readlane((unsigned int)(word >> 32), kt - chunk);
+      const unsigned int half = r & 32 ? hi : lo;
+      k = r >= 0 && ((half >> (r & 31)) & 1u) ? ~0ull : 0ull;
+    } else {
+      tile_bits(mrow, kt * 64, block, nb, r, any, k);
+    }
+    const int past = q - kt * 64;
+    if (past < 63) k &= past < 0 ? 0ull : (2ull << past) - 1ull;
+    return (unsigned int)(k >> from);
+  }
+};
+
+// All ones if bit c of bits is set, else 0 (one v_bfe_i32); x where it is, else `other` (v_bfi_b32).
+__device__ inline unsigned int bit_mask(unsigned int bits, int c) {
+  return (unsigned int)__builtin_amdgcn_sbfe((int)bits, c, 1);
+}
+__device__ inline float masked(float x, unsigned int mask, float other) {
+  return __uint_as_float((__float_as_uint(x) & mask) | (__float_as_uint(other) & ~mask));
+}
+
+// Two fp32 64 x 64 tiles side by side, 16 KB each, go from memory to LDS directly
+// (global_load_lds) while the previous pair is multiplied. 16-byte chunk c of row r sits at chunk
+// c ^ (r & 15): a ds_read_b128 phase (16 rows, one chunk) hits every bank once, and so do the 32
+// consecutive head dims of one row that a product along the columns reads 4 bytes a lane.
+// One natural copy serves both products (4-byte column reads cost one LDS cycle pair per 64-cycle
+// MFMA), so nothing is transposed on the way in. n 1000, B 4, 12 heads, block 64, top_c 4 + local 2:
+// forward 103 -> 86 us, dq 129 -> 112, dk / dv 198 -> 141 (matrix rate alone: 47, 71, 95) against
+// tiles staged through registers, twice where a transposed copy was needed.
+constexpr int kPairTile32 = 64 * 256;
+__device__ inline void issue_pair32(const char* x, int64_t xs, const char* y, int64_t ys,
+                                    int64_t r0, int64_t nrows, unsigned char* st, int w,
+                                    int lane) {
+  const float* xb = reinterpret_cast<const float*>(x);
+  const float* yb = reinterpret_cast<const float*>(y);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int r = (4 * j + w) * 4 + (lane >> 4);
+    const int64_t row = r0 + r < nrows ? r0 + r : nrows - 1;  // past the end: masked entries
+    const int col = ((lane & 15) ^ (r & 15)) * 4;
+    __builtin_amdgcn_global_load_lds(xb + row * xs + col, st + (4 * j + w) * 1024, 16, 0, 0);
+    __builtin_amdgcn_global_load_lds(yb + row * ys + col, st + kPairTile32 + (4 * j + w) * 1024,
+                                     16, 0, 0);
+  }
+}
+
+// LDS offsets of a lane's operands in such a tile, for the 32 rows from row 32 * part: `row[t]` the
+// 4 floats of head-dim steps 4 t .. 4 t + 3 of row 32 part + lo; `col[j]` element (row 32 part +
+// 8 g + 4 hi + j, head dim 32 dh + lo) for g = dh = 0 (others: col32()).
+struct PairOffsets32 {
+  uint32_t row[8], col[4];
+  __device__ PairOffsets32(int lane, int part) {
+    const int hi = lane >> 5, lo = lane & 31, r = 32 * part + lo;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) row[t] = (uint32_t)(r * 256 + (((8 * hi + t) ^ (r & 15)) * 16));
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      col[j] = (uint32_t)((32 * part + 4 * hi + j) * 256 + (((lo >> 2) ^ (4 * hi + j)) * 16) +
+                          (lo & 3) * 4);
+  }
+};
+__device__ inline float col32(const unsigned char* st, const PairOffsets32& o, int dh, int g,
+                              int j) {
+  return *reinterpret_cast<const float*>(st + o.col[j] + g * 2048 + ((dh ^ (g & 1)) * 128));
+}
+__device__ inline f32x4 row32(const unsigned char* st, const PairOffsets32& o, int t) {
+  return *reinterpret_cast<const f32x4*>(st + o.row[t]);
+}
+
 __global__ __launch_bounds__(256) void swap_fwd_kernel(SwapArgs a) {
-  __shared__ float ks[kTileFloats];  // K tile [key][d]
-  __shared__ float vt[kTileFloats];  // V tile [d][key]
+  __shared__ __attribute__((aligned(1024))) unsigned char st0[2 * kPairTile32];  // K, V tiles
+  __shared__ __attribute__((aligned(1024))) unsigned char st1[2 * kPairTile32];
+  __shared__ float ml[2 * 128];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, hi = lane >> 5, lo = lane & 31;
   const int qh = w & 1, kh = w >> 1;
   const int64_t nbh = a.B * a.Hq;
@@ -250,10 +305,10 @@ __global__ __launch_bounds__(256) void swap_fwd_kernel(SwapArgs a) {
   const int64_t qi = q0 + r;
   const bool qvalid = qi < a.n;
   float qreg[32];
-  load_row32<DT>(a.q, b * a.qsb + h * a.qsh + qi * a.qsn + 32 * hi, qvalid, qreg);
+  load_row32<SSA_F32>(a.q, b * a.qsb + h * a.qsh + qi * a.qsn + 32 * hi, qvalid, qreg);
   const unsigned long long* mrow = a.masks + (bh * a.nqt + qt) * a.nb;
-  const char* kb = a.k + (b * a.ksb + kvh * a.ksh) * dtype_size_dev<DT>();
-  const char* vb = a.v + (b * a.vsb + kvh * a.vsh) * dtype_size_dev<DT>();
+  const char* kb = a.k + (b * a.ksb + kvh * a.ksh) * 4;
+  const char* vb = a.v + (b * a.vsb + kvh * a.vsh) * 4;
   const float sl2 = a.scale_log2;
 
   float m = -INFINITY, l = 0.0f;
@@ -264,23 +319,20 @@ __global__ __launch_bounds__(256) void swap_fwd_kernel(SwapArgs a) {
     for (int e = 0; e < 16; ++e) o[x][e] = 0.0f;
   int64_t qlast = q0 + 63;
   if (qlast > a.n - 1) qlast = a.n - 1;
-  const int64_t nkt = qlast / 64 + 1;
-  for (int64_t kt = 0; kt < nkt; ++kt) {
-    const int64_t k0 = kt * 64;
-    unsigned long long any, keys;
-    tile_bits(mrow, k0, a.block, a.nb, qvalid ? r : -1, any, keys);
-    if (any == 0ull) continue;  // same words for every lane: uniform
-    __syncthreads();
-    stage_tile<DT>(kb, a.ksn, k0, a.n, ks, nullptr, tid);
-    stage_tile<DT>(vb, a.vsn, k0, a.n, nullptr, vt, tid);
-    __syncthreads();
-
+  TileCursor cur{mrow, (int)a.block, (int)a.nb, (int)(qlast / 64) + 1, -1, 0ull, 0ull};
+  const int nkt = cur.nkt;
+  const PairOffsets32 off(lane, kh);
+  auto key_bits = [&](int kt) {
+    return cur.keys(kt, qvalid ? r : -1, (int)qi, 32 * kh + 4 * hi);
+  };
+  auto compute = [&](const unsigned char* st, unsigned int keys) {
+    if (!__any(keys != 0u)) return;  // no row of the wave attends a key of its half
     f32x16 s;
 #pragma unroll
     for (int e = 0; e < 16; ++e) s[e] = 0.0f;
 #pragma unroll
     for (int t4 = 0; t4 < 8; ++t4) {
-      const f32x4 a4 = *reinterpret_cast<const f32x4*>(ks + (32 * kh + lo) * kLS + 32 * hi + 4 * t4);
+      const f32x4 a4 = row32(st, off, t4);
 #pragma unroll
       for (int j = 0; j < 4; ++j) s = mfma(a4[j], qreg[4 * t4 + j], s);
     }
@@ -288,50 +340,72 @@ __global__ __launch_bounds__(256) void swap_fwd_kernel(SwapArgs a) {
     float mx = -INFINITY;
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
-      const int kk = 32 * kh + (e >> 2) * 8 + hi * 4 + (e & 3);
-      const bool ok = ((keys >> kk) & 1ull) && (k0 + kk <= qi);
-      s[e] = ok ? s[e] * sl2 : -INFINITY;
+      s[e] = masked(s[e] * sl2, bit_mask(keys, (e >> 2) * 8 + (e & 3)), -INFINITY);
       mx = fmaxf(mx, s[e]);
     }
-    mx = pair_max(mx);
-    const float mnew = fmaxf(m, mx);
-    const float alpha = mnew == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - mnew);
+    const float mnew = fmaxf(m, pair_max(mx));
+    if (__any(mnew > m)) {
+      const float alpha = mnew > m ? __builtin_amdgcn_exp2f(m - mnew) : 1.0f;
+      l *= alpha;
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o[x][e] *= alpha;
+      m = mnew;
+    }
+    const float mref = m == -INFINITY ? 0.0f : m;
     float ps = 0.0f;
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
-      const float p = s[e] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(s[e] - mnew);
-      s[e] = p;
-      ps += p;
+      s[e] = __builtin_amdgcn_exp2f(s[e] - mref);
+      ps += s[e];
     }
-    l = l * alpha + ps;
-    m = mnew;
+    l += ps;
 #pragma unroll
-    for (int x = 0; x < 2; ++x)
+    for (int g = 0; g < 4; ++g)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) o[x][e] *= alpha;
+      for (int j = 0; j < 4; ++j)
 #pragma unroll
-    for (int dh = 0; dh < 2; ++dh)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const f32x4 a4 = *reinterpret_cast<const f32x4*>(vt + (32 * dh + lo) * kLS + 32 * kh + 8 * g + 4 * hi);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) o[dh] = mfma(a4[j], s[4 * g + j], o[dh]);
-      }
+        for (int dh = 0; dh < 2; ++dh)
+          o[dh] = mfma(col32(st + kPairTile32, off, dh, g, j), s[4 * g + j], o[dh]);
+  };
+  int kt = cur.next(0, lane);
+  unsigned int keys = 0u;
+  if (kt < nkt) {
+    keys = key_bits(kt);
+    issue_pair32(kb, a.ksn, vb, a.vsn, (int64_t)kt * 64, a.n, st0, w, lane);
+  }
+  while (kt < nkt) {
+    int nxt = cur.next(kt + 1, lane);
+    unsigned int nkeys = nxt < nkt ? key_bits(nxt) : 0u;
+    dma_barrier();  // st0 has landed for every wave; st1 is no longer read
+    if (nxt < nkt) issue_pair32(kb, a.ksn, vb, a.vsn, (int64_t)nxt * 64, a.n, st1, w, lane);
+    compute(st0, keys);
+    kt = nxt;
+    if (kt >= nkt) break;
+    keys = nkeys;
+    nxt = cur.next(kt + 1, lane);
+    nkeys = nxt < nkt ? key_bits(nxt) : 0u;
+    dma_barrier();  // st1 has landed; st0 is no longer read
+    if (nxt < nkt) issue_pair32(kb, a.ksn, vb, a.vsn, (int64_t)nxt * 64, a.n, st0, w, lane);
+    compute(st1, keys);
+    kt = nxt;
+    keys = nkeys;
   }
   l = pair_sum(l);
   // merge the two key halves: (m, l, O^T) of the kh = 1 waves through LDS
   __syncthreads();
-  float* buf = ks;  // 34 x 128 floats
+  float* buf = reinterpret_cast<float*>(st0);  // 32 x 128 floats
   const int slot = qh * 64 + lane;
   if (kh == 1) {
-    buf[slot] = m;
-    buf[128 + slot] = l;
+    ml[slot] = m;
+    ml[128 + slot] = l;
 #pragma unroll
-    for (int x = 0; x < 32; ++x) buf[(2 + x) * 128 + slot] = o[x >> 4][x & 15];
+    for (int x = 0; x < 32; ++x) buf[x * 128 + slot] = o[x >> 4][x & 15];
   }
   __syncthreads();
   if (kh == 1 || !qvalid) return;
-  const float m1 = buf[slot], l1 = buf[128 + slot];
+  const float m1 = ml[slot], l1 = ml[128 + slot];
   const float M = fmaxf(m, m1);
   const float a0 = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - M);
   const float a1 = m1 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m1 - M);
@@ -339,23 +413,21 @@ __global__ __launch_bounds__(256) void swap_fwd_kernel(SwapArgs a) {
   const float inv = 1.0f / lt;
   float of[32];
 #pragma unroll
-  for (int x = 0; x < 32; ++x) of[x] = (o[x >> 4][x & 15] * a0 + buf[(2 + x) * 128 + slot] * a1) * inv;
+  for (int x = 0; x < 32; ++x) of[x] = (o[x >> 4][x & 15] * a0 + buf[x * 128 + slot] * a1) * inv;
   const int64_t ooff = b * a.osb + h * a.osh + qi * a.osn;
 #pragma unroll
   for (int dh = 0; dh < 2; ++dh)
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       const int d0 = 32 * dh + 8 * g + 4 * hi, x = 16 * dh + 4 * g;
-      store4<DT>(a.o, ooff + d0, of[x], of[x + 1], of[x + 2], of[x + 3]);
+      store4<SSA_F32>(a.o, ooff + d0, of[x], of[x + 1], of[x + 2], of[x + 3]);
     }
   if (hi == 0) a.lse[bh * a.n + qi] = (M + log2f(lt)) * kLn2S;
 }
 
-template <int DT>
 __global__ __launch_bounds__(256, 2) void swap_dq_kernel(SwapArgs a) {
-  __shared__ float ks[kTileFloats];   // K [key][d]
-  __shared__ float vs[kTileFloats];   // V [key][d]
-  __shared__ float kt_[kTileFloats];  // K [d][key]
+  __shared__ __attribute__((aligned(1024))) unsigned char st0[2 * kPairTile32];  // K, V tiles
+  __shared__ __attribute__((aligned(1024))) unsigned char st1[2 * kPairTile32];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, hi = lane >> 5, lo = lane & 31;
   const int qh = w & 1, kh = w >> 1;
   const int64_t nbh = a.B * a.Hq;
@@ -366,13 +438,13 @@ __global__ __launch_bounds__(256, 2) void swap_dq_kernel(SwapArgs a) {
   const int64_t qi = q0 + r;
   const bool qvalid = qi < a.n;
   float qreg[32], greg[32];
-  load_row32<DT>(a.q, b * a.qsb + h * a.qsh + qi * a.qsn + 32 * hi, qvalid, qreg);
+  load_row32<SSA_F32>(a.q, b * a.qsb + h * a.qsh + qi * a.qsn + 32 * hi, qvalid, qreg);
   const int64_t ooff = b * a.osb + h * a.osh + qi * a.osn + 32 * hi;
-  load_row32<DT>(a.dout, ooff, qvalid, greg);
+  load_row32<SSA_F32>(a.dout, ooff, qvalid, greg);
   float Di;
   {
     float orow[32];
-    load_row32<DT>(a.o, ooff, qvalid, orow);
+    load_row32<SSA_F32>(a.o, ooff, qvalid, orow);
     float acc = 0.0f;
 #pragma unroll
     for (int t = 0; t < 32; ++t) acc = fmaf(greg[t], orow[t], acc);
@@ -382,8 +454,8 @@ __global__ __launch_bounds__(256, 2) void swap_dq_kernel(SwapArgs a) {
   const float lse2 = qvalid ? a.lse[rid] * kLog2eS : 0.0f;
   if (qvalid && kh == 0 && hi == 0) a.delta[rid] = Di;
   const unsigned long long* mrow = a.masks + (bh * a.nqt + qt) * a.nb;
-  const char* kb = a.k + (b * a.ksb + kvh * a.ksh) * dtype_size_dev<DT>();
-  const char* vb = a.v + (b * a.vsb + kvh * a.vsh) * dtype_size_dev<DT>();
+  const char* kb = a.k + (b * a.ksb + kvh * a.ksh) * 4;
+  const char* vb = a.v + (b * a.vsb + kvh * a.vsh) * 4;
   const float sl2 = a.scale_log2;
 
   f32x16 dqa[2];
@@ -393,17 +465,14 @@ __global__ __launch_bounds__(256, 2) void swap_dq_kernel(SwapArgs a) {
     for (int e = 0; e < 16; ++e) dqa[x][e] = 0.0f;
   int64_t qlast = q0 + 63;
   if (qlast > a.n - 1) qlast = a.n - 1;
-  const int64_t nkt = qlast / 64 + 1;
-  for (int64_t kt = 0; kt < nkt; ++kt) {
-    const int64_t k0 = kt * 64;
-    unsigned long long any, keys;
-    tile_bits(mrow, k0, a.block, a.nb, qvalid ? r : -1, any, keys);
-    if (any == 0ull) continue;
-    __syncthreads();
-    stage_tile<DT>(kb, a.ksn, k0, a.n, ks, kt_, tid);
-    stage_tile<DT>(vb, a.vsn, k0, a.n, vs, nullptr, tid);
-    __syncthreads();
-
+  TileCursor cur{mrow, (int)a.block, (int)a.nb, (int)(qlast / 64) + 1, -1, 0ull, 0ull};
+  const int nkt = cur.nkt;
+  const PairOffsets32 off(lane, kh);
+  auto key_bits = [&](int kt) {
+    return cur.keys(kt, qvalid ? r : -1, (int)qi, 32 * kh + 4 * hi);
+  };
+  auto compute = [&](const unsigned char* st, unsigned int keys) {
+    if (!__any(keys != 0u)) return;  // no row of the wave attends a key of its half
     f32x16 s, dp;
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
@@ -412,8 +481,8 @@ __global__ __launch_bounds__(256, 2) void swap_dq_kernel(SwapArgs a) {
     }
 #pragma unroll
     for (int t4 = 0; t4 < 8; ++t4) {
-      const f32x4 a4 = *reinterpret_cast<const f32x4*>(ks + (32 * kh + lo) * kLS + 32 * hi + 4 * t4);
-      const f32x4 b4 = *reinterpret_cast<const f32x4*>(vs + (32 * kh + lo) * kLS + 32 * hi + 4 * t4);
+      const f32x4 a4 = row32(st, off, t4);
+      const f32x4 b4 = row32(st + kPairTile32, off, t4);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         s = mfma(a4[j], qreg[4 * t4 + j], s);
@@ -422,22 +491,43 @@ __global__ __launch_bounds__(256, 2) void swap_dq_kernel(SwapArgs a) {
     }
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
-      const int kk = 32 * kh + (e >> 2) * 8 + hi * 4 + (e & 3);
-      const bool ok = ((keys >> kk) & 1ull) && (k0 + kk <= qi);
-      const float p = ok ? __builtin_amdgcn_exp2f(fmaf(s[e], sl2, -lse2)) : 0.0f;
+      const float p = masked(__builtin_amdgcn_exp2f(fmaf(s[e], sl2, -lse2)),
+                             bit_mask(keys, (e >> 2) * 8 + (e & 3)), 0.0f);
       s[e] = p * (dp[e] - Di);  // dS^T
     }
 #pragma unroll
-    for (int dh = 0; dh < 2; ++dh)
+    for (int g = 0; g < 4; ++g)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const f32x4 a4 = *reinterpret_cast<const f32x4*>(kt_ + (32 * dh + lo) * kLS + 32 * kh + 8 * g + 4 * hi);
+      for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) dqa[dh] = mfma(a4[j], s[4 * g + j], dqa[dh]);
-      }
+        for (int dh = 0; dh < 2; ++dh)
+          dqa[dh] = mfma(col32(st, off, dh, g, j), s[4 * g + j], dqa[dh]);
+  };
+  int kt = cur.next(0, lane);
+  unsigned int keys = 0u;
+  if (kt < nkt) {
+    keys = key_bits(kt);
+    issue_pair32(kb, a.ksn, vb, a.vsn, (int64_t)kt * 64, a.n, st0, w, lane);
+  }
+  while (kt < nkt) {
+    int nxt = cur.next(kt + 1, lane);
+    unsigned int nkeys = nxt < nkt ? key_bits(nxt) : 0u;
+    dma_barrier();  // st0 has landed for every wave; st1 is no longer read
+    if (nxt < nkt) issue_pair32(kb, a.ksn, vb, a.vsn, (int64_t)nxt * 64, a.n, st1, w, lane);
+    compute(st0, keys);
+    kt = nxt;
+    if (kt >= nkt) break;
+    keys = nkeys;
+    nxt = cur.next(kt + 1, lane);
+    nkeys = nxt < nkt ? key_bits(nxt) : 0u;
+    dma_barrier();  // st1 has landed; st0 is no longer read
+    if (nxt < nkt) issue_pair32(kb, a.ksn, vb, a.vsn, (int64_t)nxt * 64, a.n, st0, w, lane);
+    compute(st1, keys);
+    kt = nxt;
+    keys = nkeys;
   }
   __syncthreads();
-  float* buf = ks;  // 32 x 128 floats
+  float* buf = reinterpret_cast<float*>(st0);  // 32 x 128 floats
   const int slot = qh * 64 + lane;
   if (kh == 1) {
 #pragma unroll
@@ -488,13 +578,10 @@ __device__ inline int64_t next_active_tile(const SwapArgs& a, int64_t bh, int64_
   return a.nqt;
 }
 
-template <int DT>
 __global__ __launch_bounds__(256, 2) void swap_dkdv_kernel(SwapArgs a) {
-  __shared__ float qs[kTileFloats];   // Q [q][d]
-  __shared__ float gs[kTileFloats];   // dO [q][d]
-  __shared__ float qtT[kTileFloats];  // Q [d][q]
-  __shared__ float gtT[kTileFloats];  // dO [d][q]
-  __shared__ float lse_s[64], del_s[64];
+  __shared__ __attribute__((aligned(1024))) unsigned char st0[2 * kPairTile32];  // Q, dO tiles
+  __shared__ __attribute__((aligned(1024))) unsigned char st1[2 * kPairTile32];
+  __shared__ float ld_s[2][2][64];  // [stage][lse, delta][row]
   __shared__ unsigned long long act_s[4];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, hi = lane >> 5, lo = lane & 31;
   const int kq = w & 1, qp = w >> 1;
@@ -505,8 +592,8 @@ __global__ __launch_bounds__(256, 2) void swap_dkdv_kernel(SwapArgs a) {
   const int64_t key = k0 + 32 * kq + lo;
   const bool kvalid = key < a.n;
   float kreg[32], vreg[32];
-  load_row32<DT>(a.k, b * a.ksb + kvh * a.ksh + key * a.ksn + 32 * hi, kvalid, kreg);
-  load_row32<DT>(a.v, b * a.vsb + kvh * a.vsh + key * a.vsn + 32 * hi, kvalid, vreg);
+  load_row32<SSA_F32>(a.k, b * a.ksb + kvh * a.ksh + key * a.ksn + 32 * hi, kvalid, kreg);
+  load_row32<SSA_F32>(a.v, b * a.vsb + kvh * a.vsh + key * a.vsn + 32 * hi, kvalid, vreg);
   const int64_t ck = kvalid ? key / a.block : 0;
   const float sl2 = a.scale_log2;
 
@@ -518,69 +605,104 @@ __global__ __launch_bounds__(256, 2) void swap_dkdv_kernel(SwapArgs a) {
       dka[x][e] = 0.0f;
       dva[x][e] = 0.0f;
     }
-  for (int64_t g = 0; g < a.G; ++g) {
-    const int64_t hq = kvh * a.G + g, bh = b * a.Hq + hq;
-    const char* qb = a.q + (b * a.qsb + hq * a.qsh) * dtype_size_dev<DT>();
-    const char* gb = a.dout + (b * a.osb + hq * a.osh) * dtype_size_dev<DT>();
-    int64_t chunk = -1;
-    for (int64_t qt = next_active_tile(a, bh, k0, k0 / 64, act_s, chunk); qt < a.nqt;
-         qt = next_active_tile(a, bh, k0, qt + 1, act_s, chunk)) {
-      const unsigned long long* mrow = a.masks + (bh * a.nqt + qt) * a.nb;
-      const unsigned long long mw = kvalid ? mrow[ck] : 0ull;
-      const int64_t q0 = qt * 64;
-      __syncthreads();
-      stage_tile<DT>(qb, a.qsn, q0, a.n, qs, qtT, tid);
-      stage_tile<DT>(gb, a.osn, q0, a.n, gs, gtT, tid);
-      if (tid < 64) {
-        const bool ok = q0 + tid < a.n;
-        lse_s[tid] = ok ? a.lse[bh * a.n + q0 + tid] * kLog2eS : 0.0f;
-        del_s[tid] = ok ? a.delta[bh * a.n + q0 + tid] : 0.0f;
-      }
-      __syncthreads();
-
-      f32x16 s, dp;
+  const PairOffsets32 off(lane, qp);
+  auto compute = [&](const unsigned char* st, const float (*ld)[64], unsigned int rows) {
+    if (!__any(rows != 0u)) return;  // no row of the wave's half attends a key of its half
+    f32x16 s, dp;
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        s[e] = 0.0f;
-        dp[e] = 0.0f;
-      }
-#pragma unroll
-      for (int t4 = 0; t4 < 8; ++t4) {
-        const f32x4 a4 = *reinterpret_cast<const f32x4*>(qs + (32 * qp + lo) * kLS + 32 * hi + 4 * t4);
-        const f32x4 b4 = *reinterpret_cast<const f32x4*>(gs + (32 * qp + lo) * kLS + 32 * hi + 4 * t4);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          s = mfma(a4[j], kreg[4 * t4 + j], s);
-          dp = mfma(b4[j], vreg[4 * t4 + j], dp);
-        }
-      }
-      // query row of register e: 32*qp + (e/4)*8 + hi*4 + e%4 of the tile
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int qq = 32 * qp + (e >> 2) * 8 + hi * 4 + (e & 3);
-        const bool ok = ((mw >> qq) & 1ull) && (key <= q0 + qq);
-        const float p = ok ? __builtin_amdgcn_exp2f(fmaf(s[e], sl2, -lse_s[qq])) : 0.0f;
-        s[e] = p;
-        dp[e] = p * (dp[e] - del_s[qq]);  // dS
-      }
-#pragma unroll
-      for (int dh = 0; dh < 2; ++dh)
-#pragma unroll
-        for (int g4 = 0; g4 < 4; ++g4) {
-          const int off = (32 * dh + lo) * kLS + 32 * qp + 8 * g4 + 4 * hi;
-          const f32x4 ga = *reinterpret_cast<const f32x4*>(gtT + off);
-          const f32x4 qa = *reinterpret_cast<const f32x4*>(qtT + off);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            dva[dh] = mfma(ga[j], s[4 * g4 + j], dva[dh]);
-            dka[dh] = mfma(qa[j], dp[4 * g4 + j], dka[dh]);
-          }
-        }
+    for (int e = 0; e < 16; ++e) {
+      s[e] = 0.0f;
+      dp[e] = 0.0f;
     }
+#pragma unroll
+    for (int t4 = 0; t4 < 8; ++t4) {
+      const f32x4 a4 = row32(st, off, t4);
+      const f32x4 b4 = row32(st + kPairTile32, off, t4);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        s = mfma(a4[j], kreg[4 * t4 + j], s);
+        dp = mfma(b4[j], vreg[4 * t4 + j], dp);
+      }
+    }
+    // query row of register e: 32*qp + (e/4)*8 + hi*4 + e%4 of the tile
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int qq = 32 * qp + (e >> 2) * 8 + hi * 4 + (e & 3);
+      s[e] = masked(__builtin_amdgcn_exp2f(fmaf(s[e], sl2, -ld[0][qq])),
+                    bit_mask(rows, (e >> 2) * 8 + (e & 3)), 0.0f);
+      dp[e] = s[e] * (dp[e] - ld[1][qq]);  // dS
+    }
+#pragma unroll
+    for (int g4 = 0; g4 < 4; ++g4)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int dh = 0; dh < 2; ++dh) {
+          dva[dh] = mfma(col32(st + kPairTile32, off, dh, g4, j), s[4 * g4 + j], dva[dh]);
+          dka[dh] = mfma(col32(st, off, dh, g4, j), dp[4 * g4 + j], dka[dh]);
+        }
+  };
+  // The walk over (query head, query tile) pairs. A pair's mask word and (threads 0..127) its row's
+  // lse or delta are loaded one pair before its tiles are, two before it is multiplied.
+  struct Pair {
+    int64_t g, qt;
+    unsigned long long mw;
+    float ld;
+  };
+  int64_t chunk = -1;
+  auto next_pair = [&](Pair at) {  // the pair at or after `at`; g == G: none left
+    for (; at.g < a.G; ++at.g, at.qt = k0 / 64, chunk = -1) {
+      const int64_t bh = b * a.Hq + kvh * a.G + at.g;
+      at.qt = next_active_tile(a, bh, k0, at.qt, act_s, chunk);
+      if (at.qt < a.nqt) {
+        at.mw = kvalid ? a.masks[(bh * a.nqt + at.qt) * a.nb + ck] : 0ull;
+        const int64_t row = at.qt * 64 + lane;
+        if (tid < 128)  // (rows past the end belong to no list: any finite value will do)
+          at.ld = (tid < 64 ? a.lse : a.delta)[bh * a.n + (row < a.n ? row : a.n - 1)];
+        break;
+      }
+    }
+    return at;
+  };
+  auto after = [&](Pair at) {
+    if (at.g >= a.G) return at;
+    ++at.qt;
+    return next_pair(at);
+  };
+  auto issue = [&](const Pair& at, unsigned char* st, float (*ld)[64]) {
+    const int64_t hq = kvh * a.G + at.g;
+    issue_pair32(a.q + (b * a.qsb + hq * a.qsh) * 4, a.qsn, a.dout + (b * a.osb + hq * a.osh) * 4,
+                 a.osn, at.qt * 64, a.n, st, w, lane);
+    if (tid < 128) ld[tid >> 6][lane] = tid < 64 ? at.ld * kLog2eS : at.ld;
+  };
+  // the rows of the lane's half that attend its key, as the 32 bits from row 32 qp + 4 hi on
+  auto rows_of = [&](const Pair& at) {
+    unsigned long long mw = at.mw;
+    const int ahead = (int)(key - at.qt * 64);  // token causal: rows at or after the key
+    if (ahead > 0) mw &= ~0ull << ahead;        // (< 64: the walk starts at the key's tile)
+    return (unsigned int)(mw >> (32 * qp + 4 * hi));
+  };
+  Pair at = next_pair(Pair{0, k0 / 64, 0ull, 0.0f});
+  if (at.g < a.G) issue(at, st0, ld_s[0]);
+  Pair nx = after(at);
+  while (at.g < a.G) {
+    dma_barrier();  // stage 0 has landed for every wave; stage 1 is no longer read
+    if (nx.g < a.G) issue(nx, st1, ld_s[1]);
+    Pair nn = after(nx);
+    compute(st0, ld_s[0], rows_of(at));
+    at = nx;
+    nx = nn;
+    if (at.g >= a.G) break;
+    dma_barrier();  // stage 1 has landed; stage 0 is no longer read
+    if (nx.g < a.G) issue(nx, st0, ld_s[0]);
+    nn = after(nx);
+    compute(st1, ld_s[1], rows_of(at));
+    at = nx;
+    nx = nn;
   }
   __syncthreads();
-  float* bk = qs;  // 32 x 128 floats each
-  float* bv = gs;
+  float* bk = reinterpret_cast<float*>(st0);  // 32 x 128 floats each
+  float* bv = reinterpret_cast<float*>(st1);
   const int slot = kq * 64 + lane;
   if (qp == 1) {
 #pragma unroll
@@ -701,55 +823,6 @@ __device__ inline u32x4 lds_cols(const unsigned char* st, const PairOffsets& o, 
   const uint2 x = lds_read_tr(st + o.col[dh][0] + 2048 * u);
   const uint2 y = lds_read_tr(st + o.col[dh][1] + 2048 * u);
   return u32x4{x.x, x.y, y.x, y.y};
-}
-
-// Cursor over the key tiles of a query tile that hold a selected key: lane t tests tile 64 c + t,
-// one round of loads per 64 tiles. The same in every wave of the workgroup.
-struct TileCursor {
-  const unsigned long long* mrow;
-  int block, nb, nkt, chunk;
-  unsigned long long act, word;  // word: this lane's tile's rows (any of its blocks)
-  __device__ int next(int kt, int lane) {
-    while (kt < nkt) {
-      const int c0 = kt & ~63;
-      if (c0 != chunk) {
-        unsigned long long any = 0ull, unused;
-        if (c0 + lane < nkt) tile_bits(mrow, (c0 + lane) * 64, block, nb, -1, any, unused);
-        act = __ballot(any != 0ull);
-        word = any;
-        chunk = c0;
-      }
-      const unsigned long long rest = act & (~0ull << (kt - c0));
-      if (rest != 0ull) return c0 + __builtin_ctzll(rest);
-      kt = c0 + 64;
-    }
-    return nkt;
-  }
-  // the keys of tile kt (the last next()) that row r of the query tile attends, at most key row q
-  // (r < 0: none), as the 32 bits from key `from` on. A tile inside one block (block a multiple of
-  // 64) needs only the word next() loaded, read from its lane: no memory wait per tile.
-  __device__ unsigned int keys(int kt, int r, int q, int from) const {
-    unsigned long long any, k;
-    if (block % 64 == 0) {
-      const unsigned int lo = __builtin_amdgcn_readlane((unsigned int)word, kt - chunk);
-      const unsigned int hi = __builtin_amdgcn_readlane((unsigned int)(word >> 32), kt - chunk);
-      const unsigned int half = r & 32 ? hi : lo;
-      k = r >= 0 && ((half >> (r & 31)) & 1u) ? ~0ull : 0ull;
-    } else {
-      tile_bits(mrow, kt * 64, block, nb, r, any, k);
-    }
-    const int past = q - kt * 64;
-    if (past < 63) k &= past < 0 ? 0ull : (2ull << past) - 1ull;
-    return (unsigned int)(k >> from);
-  }
-};
-
-// All ones if bit c of bits is set, else 0 (one v_bfe_i32); x where it is, else `other` (v_bfi_b32).
-__device__ inline unsigned int bit_mask(unsigned int bits, int c) {
-  return (unsigned int)__builtin_amdgcn_sbfe((int)bits, c, 1);
-}
-__device__ inline float masked(float x, unsigned int mask, float other) {
-  return __uint_as_float((__float_as_uint(x) & mask) | (__float_as_uint(other) & ~mask));
 }
 
 // one row's 32 halves [32*hi, 32*hi + 32) as 4 packed operands (zeros when !valid)
@@ -1214,7 +1287,7 @@ int masked_tiled_fwd(const void* q, const void* k, const void* v, void* out, flo
   const unsigned grid = (unsigned)(B * Hq * a.nqt);
   row_block_masks_kernel<<<grid, 256, 0, st>>>(a);
   SSA_TRY(launch_status("row_block_masks_kernel"));
-  if (dtype == SSA_F32) swap_fwd_kernel<SSA_F32><<<grid, 256, 0, st>>>(a);
+  if (dtype == SSA_F32) swap_fwd_kernel<<<grid, 256, 0, st>>>(a);
   else if (dtype == SSA_F16) swap_fwd16_kernel<SSA_F16><<<grid, 256, 0, st>>>(a);
   else swap_fwd16_kernel<SSA_BF16><<<grid, 256, 0, st>>>(a);
   return launch_status("swap_fwd_kernel");
@@ -1243,8 +1316,8 @@ int masked_tiled_bwd(const void* q, const void* k, const void* v, const void* ou
     SSA_TRY(launch_status("row_block_masks_kernel"));
   }
   if (dtype == SSA_F32) {
-    swap_dq_kernel<SSA_F32><<<gq, 256, 0, st>>>(a);
-    swap_dkdv_kernel<SSA_F32><<<gk, 256, 0, st>>>(a);
+    swap_dq_kernel<<<gq, 256, 0, st>>>(a);
+    swap_dkdv_kernel<<<gk, 256, 0, st>>>(a);
   } else if (dtype == SSA_F16) {
     swap_dq16_kernel<SSA_F16><<<gq, 256, 0, st>>>(a);
     swap_dkdv16_kernel<SSA_F16><<<gk, 256, 0, st>>>(a);
