@@ -382,6 +382,116 @@ __device__ inline void block_partial(const DecodeParams& p, float* part, float* 
   }
 }
 
+// block_partial for 16-bit caches at head dim 128, of one wave of a workgroup: a load instruction
+// reads four whole 256-byte rows (lane: 16-byte chunk lane & 15 of key group lane / 16), 32 keys of
+// K and of V at a time, both in flight before the scores are formed. Three halving exchanges and a
+// sum over the 16 lanes of a key group leave each pair of lanes the dot of one key; their exps go
+// to ps. The general path walks a key row per lane, one 16-byte load after the other. With the
+// survivors' LDS sized by the step (two workgroups a CU instead of one): 8 sequences x 32 heads,
+// 32.7K tokens, 18 blocks of 128: 127 -> 109 us a launch (2.9 TB/s). What bounds it now is the
+// merge each workgroup starts with, which has no loads in flight.
+template <int DT>
+__device__ inline void block_partial_128(const DecodeParams& p, float* part, float* qs, float* ps,
+                                         int64_t b, int64_t h, int64_t kvh, int64_t pos, int64_t c,
+                                         int64_t kofs, int64_t kcnt) {
+  constexpr int D = 128, T = 8;
+  const int lane = threadIdx.x & 63, kg = lane >> 4, ch = lane & 15;
+  const int64_t key0 = c * p.block + kofs;
+  int64_t key1 = c * p.block + p.block;
+  if (key0 + kcnt < key1) key1 = key0 + kcnt;
+  if (key1 > pos + 1) key1 = pos + 1;
+  if (key1 > p.cap) key1 = p.cap;
+  const int nk = (int)(key1 - key0);
+  if (nk <= 0) {
+    if (lane == 0) {
+      part[0] = -INFINITY;
+      part[1] = 0.0f;
+    }
+    for (int e = lane; e < D; e += 64) part[2 + e] = 0.0f;
+    return;
+  }
+  const int64_t newkey = p.fused_append ? pos : -1;
+  const unsigned short* kb = reinterpret_cast<const unsigned short*>(p.k) + b * p.ksb + kvh * p.ksh;
+  const unsigned short* vb = reinterpret_cast<const unsigned short*>(p.v) + b * p.vsb + kvh * p.vsh;
+  const unsigned short* kn = reinterpret_cast<const unsigned short*>(p.k_new) + b * p.knb + kvh * p.knh;
+  const unsigned short* vn = reinterpret_cast<const unsigned short*>(p.v_new) + b * p.vnb + kvh * p.vnh;
+  const int64_t qoff = b * p.qsb + h * p.qsh;
+  const float q0 = load_elem<DT>(p.q, qoff + lane), q1 = load_elem<DT>(p.q, qoff + 64 + lane);
+  float m = -INFINITY, l = 0.0f, acc[8], qv[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) acc[e] = 0.0f;
+  for (int k0 = 0; k0 < nk; k0 += 4 * T) {
+    u32x4 kx[T], vx[T];
+#pragma unroll
+    for (int t = 0; t < T; ++t) {  // (past the range: its last key, weight 0)
+      const int kk = k0 + kg + 4 * t < nk ? k0 + kg + 4 * t : nk - 1;
+      const int64_t key = key0 + kk;
+      kx[t] = *reinterpret_cast<const u32x4*>((key == newkey ? kn : kb + key * p.ksn) + ch * 8);
+      vx[t] = *reinterpret_cast<const u32x4*>((key == newkey ? vn : vb + key * p.vsn) + ch * 8);
+    }
+    if (k0 == 0) {  // the query row, staged behind the loads
+      qs[lane] = q0;
+      qs[64 + lane] = q1;
+      wave_lds_sync();
+#pragma unroll
+      for (int e = 0; e < 8; ++e) qv[e] = qs[8 * ch + e];
+    }
+    float sc[T];
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      float x[8];
+      unpack8(kx[t], x, DT == SSA_BF16);
+      float a = 0.0f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) a = fmaf(qv[e], x[e], a);
+      sc[t] = a;
+    }
+#pragma unroll
+    for (int w = 8; w >= 2; w >>= 1) {  // keep the half of the values whose t bit = ch bit w
+      const bool hi = (ch & w) != 0;
+#pragma unroll
+      for (int i = 0; i < w / 2; ++i) {
+        const float keep = hi ? sc[i + w / 2] : sc[i];
+        const float send = hi ? sc[i] : sc[i + w / 2];
+        sc[i] = keep + lane_xor(send, w);
+      }
+    }
+    const float s = (sc[0] + lane_xor(sc[0], 1)) * p.scale_log2;  // key k0 + kg + 4 (ch >> 1)
+    const int mine = k0 + kg + 4 * (ch >> 1);
+    const float mnew = fmaxf(m, wave_max(mine < nk ? s : -INFINITY));  // (key k0 is in range)
+    const float alpha = exp2f(m - mnew);
+    m = mnew;
+    const float pk = mine < nk ? exp2f(s - mnew) : 0.0f;
+    wave_lds_sync();  // the previous 32 keys' weights have been read
+    if ((ch & 1) == 0) ps[kg + 4 * (ch >> 1)] = pk;
+    l = l * alpha + ((ch & 1) == 0 ? pk : 0.0f);
+    wave_lds_sync();
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] *= alpha;
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      float x[8];
+      unpack8(vx[t], x, DT == SSA_BF16);
+      const float w = ps[kg + 4 * t];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[e] = fmaf(w, x[e], acc[e]);
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    acc[e] += lane_xor(acc[e], 16);
+    acc[e] += lane_xor(acc[e], 32);
+  }
+  if (kg == 0)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) part[2 + 8 * ch + e] = acc[e];
+  l = wave_sum(l);
+  if (lane == 0) {
+    part[0] = m;
+    part[1] = l;
+  }
+}
+
 // grid (B*Hq*nq), 4 waves per row: wave w merges partials [w * q, (w + 1) * q) of the row (q =
 // ceil(cnt / 4)) with the usual max-rescaling, loading 8 partial rows at a time (one memory
 // latency per batch, not per partial); the waves' sums are then added through LDS.
@@ -537,6 +647,7 @@ struct FusedStep {
   int64_t B, Hq, Hkv, G, d, nbk, ncand, K, local, pos, block, W;
   float coef2;
   int nchunk, ngroups;
+  int lseg;  // attend_segment_log2(nchunk, 8)
   unsigned int* arrive;  // (B*Hq) arrival counters
   unsigned int* ckth;    // (B*Hq, nchunk): entries the chunk kept (min(K, its candidates))
   unsigned int* ckey;    // (B*Hq, nchunk, kDTop): the chunk's kept keys, best first, then 0
@@ -697,18 +808,35 @@ __device__ inline unsigned int wave_sort_asc(unsigned int v) {
   return v;
 }
 
+// log2 of the entries of one wave's segment of survivors: a wave holds the lists of every NWA-th
+// chunk (rounded up to a power of two: the merge addresses segments by shifts).
+__host__ __device__ inline int attend_segment_log2(int nchunk, int nwa) {
+  int lg = 0;
+  while ((nwa << lg) < nchunk) ++lg;
+  return lg + 6;  // kDTop = 64 entries a chunk
+}
+static_assert(kDTop == 64, "attend_segment_log2");
+
 // One attend workgroup's work (NWA waves): group `group` of the selected slots of query row
 // `row` (b*Hq + h), NWA / HALVES slots, each attended by HALVES waves (a wave per 1/HALVES of
 // the block's keys, each storing a partial of its own).
-template <int DT, int NWA, int HALVES>
+template <int DT, int NWA, int HALVES, bool D128, bool LONG>
 __device__ inline void attend_group(const FusedStep& f, const DecodeParams& p, int64_t row,
                                     int64_t group) {
   constexpr int NT = NWA * 64, SPW = NWA / HALVES;
-  __shared__ unsigned int skey[kDSurv], sidx[kDSurv];
+  // survivors of the merge, a segment per wave: as many entries as this step's chunk lists hold
+  // (attend_lds), not the most there can be (64 KB, which left one workgroup on a CU whatever the
+  // context). LONG (the most, more than 64 chunks): a fixed array, which the merge addresses
+  // faster: 25.3 us a step against 25.7 at 8192 blocks
+  extern __shared__ unsigned int dyn_lds[];
+  __shared__ unsigned int held[LONG ? 2 * kDSurv : 1];
+  const int lseg = LONG ? 10 : f.lseg;
+  unsigned int* skey = LONG ? held : dyn_lds;
+  unsigned int* sidx = skey + (NWA << lseg);
   __shared__ unsigned int sel[kDBitWords], tie[kDBitWords];
   __shared__ int32_t list[kDMaxW];
   __shared__ __attribute__((aligned(16))) float qs[NWA][kDMaxD];
-  __shared__ float ps[NWA][kDMaxBlock];
+  __shared__ float ps[NWA][kDMaxBlock / HALVES];
   __shared__ float wgt[kDMaxW];
   __shared__ float wpart[NWA][kDMaxD + 2];  // the waves' partials, combined into the group's
   __shared__ unsigned int red[NWA], rand_[4], hist[256];  // (hist: also reduction scratch)
@@ -742,7 +870,6 @@ __device__ inline void attend_group(const FusedStep& f, const DecodeParams& p, i
   const int64_t K = f.K;
   const int nch = f.nchunk;
   const int ne = nch * kDTop;
-  constexpr int SEG = kDSurv / NWA;
   auto merge_pass = [&](auto pc) -> bool {
     constexpr int P = decltype(pc)::value, CPR = 64 / P;
     constexpr int KR = (kDSurv / kDTop + NWA * CPR - 1) / (NWA * CPR);
@@ -798,7 +925,7 @@ __device__ inline void attend_group(const FusedStep& f, const DecodeParams& p, i
       const bool take = kk[u] >= floor_;
       const unsigned long long bt = __ballot(take);
       if (take) {
-        const int sl = wv * SEG + at + (int)__popcll(bt & lt);
+        const int sl = (wv << lseg) + at + (int)__popcll(bt & lt);
         skey[sl] = kk[u];
         sidx[sl] = ci[u];
       }
@@ -823,7 +950,7 @@ __device__ inline void attend_group(const FusedStep& f, const DecodeParams& p, i
     int base = 0;
 #pragma unroll
     for (int v = 0; v < NWA; ++v) base = v == w ? pre[v] : base;
-    return w * SEG + (i - base);
+    return (w << lseg) + (i - base);
   };
   // one wave (J survivors per lane): K-th key, ties by lowest block, then the ascending list of
   // the taken blocks, own block and local predecessors -- no workgroup barrier until the list is
@@ -1002,8 +1129,11 @@ __device__ inline void attend_group(const FusedStep& f, const DecodeParams& p, i
   float* prow = p.part + row * f.ngroups * stride;
   if (s < num) {
     const int64_t kh = (f.block + HALVES - 1) / HALVES;
-    block_partial<DT, true, 16 / HALVES, false>(p, wpart[wv], qs[wv], ps[wv], b, h, kvh, 0, pos,
-                                                list[s], half * kh, kh);
+    if constexpr (D128)
+      block_partial_128<DT>(p, wpart[wv], qs[wv], ps[wv], b, h, kvh, pos, list[s], half * kh, kh);
+    else
+      block_partial<DT, true, 16 / HALVES, false>(p, wpart[wv], qs[wv], ps[wv], b, h, kvh, 0, pos,
+                                                  list[s], half * kh, kh);
   } else {
     if (lane == 0) {
       wpart[wv][0] = -INFINITY;
@@ -1128,9 +1258,9 @@ __device__ inline void attend_group(const FusedStep& f, const DecodeParams& p, i
 }
 
 // 8 waves: 4 slots, each attended by 2 waves (half of the block's keys each)
-template <int DT>
+template <int DT, bool D128, bool LONG>
 __global__ __launch_bounds__(512) void decode_attend_fused_kernel(FusedStep f, DecodeParams p) {
-  attend_group<DT, 8, 2>(f, p, blockIdx.y, blockIdx.x);
+  attend_group<DT, 8, 2, D128, LONG>(f, p, blockIdx.y, blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1527,6 +1657,8 @@ int decode_step_impl(const void* q, const void* k_new, const void* v_new, void* 
     f.cidx = reinterpret_cast<unsigned int*>(ws + f_arrive + f_kth + f_list);
     f.kv_num = kv_num;
     f.kv_idx = kv_idx;
+    f.lseg = attend_segment_log2(f.nchunk, 8);
+    const size_t alds = ((size_t)8 << f.lseg) * 8;  // (key, block) per entry
     const dim3 g1((unsigned)nchunk, (unsigned)(B * Hkv)), g2((unsigned)f.ngroups, (unsigned)(B * Hq));
 #define SSA_FUSED_ROUTE(DT, NW, NWT)                                                              \
   do {                                                                                            \
@@ -1539,7 +1671,12 @@ int decode_step_impl(const void* q, const void* k_new, const void* v_new, void* 
     if (chunk == kDChunk) SSA_FUSED_ROUTE(DT, 16, 16);                                            \
     else if (chunk == kDChunk / 4) SSA_FUSED_ROUTE(DT, 4, 8);                                     \
     else SSA_FUSED_ROUTE(DT, 8, 8);                                                               \
-    decode_attend_fused_kernel<DT><<<g2, 512, 0, st>>>(f, p);                                     \
+    constexpr bool w = DT != SSA_F32;                                                             \
+    if (w && d == 128 && f.lseg < 10)                                                             \
+      decode_attend_fused_kernel<DT, w, false><<<g2, 512, alds, st>>>(f, p);                      \
+    else if (w && d == 128) decode_attend_fused_kernel<DT, w, true><<<g2, 512, 0, st>>>(f, p);    \
+    else if (f.lseg < 10) decode_attend_fused_kernel<DT, false, false><<<g2, 512, alds, st>>>(f, p); \
+    else decode_attend_fused_kernel<DT, false, true><<<g2, 512, 0, st>>>(f, p);                   \
   } while (0)
     switch (dtype) {
       case SSA_F32: SSA_FUSED_STEP(SSA_F32); break;

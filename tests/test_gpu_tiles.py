@@ -146,3 +146,36 @@ def test_masked_attention_tiles_match_oracle(cuda, dtype, hq, hkv, n, block, top
     assert np.abs(np_of(out) - ref).max() < tol
     for got, want in zip(grads, O.masked_grads(q, k, v, lists, g, block)):
         assert np.abs(np_of(got) - want).max() < tol * max(1.0, np.abs(want).max())
+
+
+# routed decode step: head dim 128 over parts of a block of less, exactly and more than 32 keys, the
+# new token first and last in its block; contexts whose chunk lists fill one, two and four segments
+# and all of the longest (more than 64 chunks: 4200 blocks), at head dim 64 too
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("d,block,n,top_c", [(128, 16, 33, 2), (128, 64, 640, 4),
+                                             (128, 512, 1800, 2), (128, 128, 131072, 8),
+                                             (64, 128, 66000, 64), (128, 16, 67196, 64),
+                                             (64, 16, 67196, 64)])
+def test_decode_step_tiles_match_oracle(cuda, dtype, d, block, n, top_c):
+    """Selections exact; outputs within the bars of the decode tests (2e-2, fp32 1e-5)."""
+    from ssa_amd.ivf_decode import RoutedDecoder
+    rng = np.random.default_rng(n + d)
+    hq, hkv, steps = 4, 2, 3
+    k, v = (WL.round_to(rng.standard_normal((1, hkv, n + steps, d)).astype(np.float32), dtype)
+            for _ in range(2))
+    q = WL.round_to(rng.standard_normal((steps, 1, hq, d)).astype(np.float32), dtype)
+    kt, vt, qt = (WL.to_device(a, dtype, cuda) for a in (k, v, q))
+    dec = RoutedDecoder(1, hq, hkv, d, n + steps, block=block, top_c=top_c, local=1, dtype=dtype,
+                        device=cuda)
+    dec.prefill(kt[:, :, :n], vt[:, :, :n])
+    tol = 1e-5 if dtype == torch.float32 else 2e-2
+    for t in range(steps):
+        out = np_of(dec.step(qt[t], kt[:, :, n + t], vt[:, :, n + t]))
+        on, oi = O.route_query(q[t][:, :, None], k, block, n + t, top_c=top_c, local=1,
+                               kv_len=n + t + 1)
+        kn, ki = dec.kv_num.cpu().numpy(), dec.kv_idx.cpu().numpy()
+        for h in range(hq):
+            sel = oi[0, h, 0, :on[0, h, 0]].tolist()
+            assert ki[0, h, :kn[0, h]].tolist() == sel, (t, h)
+            ref = O.decode_attend(q[t][0, h], k[0, h // 2], v[0, h // 2], sel, n + t, block)
+            assert np.abs(out[0, h] - ref).max() < tol, (t, h)
