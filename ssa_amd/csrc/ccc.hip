@@ -400,19 +400,10 @@ int ccc_assign_rows(const float* x, int64_t m, int64_t base, int64_t d, const fl
                     int64_t nlist, unsigned long long* pbest, int64_t pcap, int32_t* assign,
                     float* rc, hipStream_t s) {
   if (m <= 0) return SSA_OK;
-  const int64_t stiles = (m + 2 * kScoreTile - 1) / (2 * kScoreTile);
-  const int64_t gmax = (nlist + kAssignC - 1) / kAssignC;
-  int64_t g = (2048 + stiles - 1) / stiles;
-  g = g > gmax ? gmax : g;
-  g = g > pcap / m ? pcap / m : g;
-  g = g < 1 ? 1 : g;
-  const int64_t per_group = (nlist + g - 1) / g;
-  const int64_t groups = (nlist + per_group - 1) / per_group;
-  ivf_score_kernel<<<dim3((unsigned)stiles, 1, (unsigned)groups), kScoreTile,
-                     kAssignC * d * sizeof(double), s>>>(x, cent, m, d, nlist, per_group, pbest);
-  SSA_TRY(launch_status("ivf_score_kernel"));
-  ccc_assign_kernel<<<(unsigned)((m + 255) / 256), 256, 0, s>>>(pbest, groups, m, base, x, cent, d,
-                                                                 assign, rc);
+  const ScoreSplit split(m, 1, nlist, pcap / m);
+  SSA_TRY(ivf_score(x, cent, 1, m, d, nlist, split, pbest, s));
+  ccc_assign_kernel<<<(unsigned)((m + 255) / 256), 256, 0, s>>>(pbest, split.groups, m, base, x,
+                                                                 cent, d, assign, rc);
   return launch_status("ccc_assign_kernel");
 }
 

@@ -26,17 +26,13 @@ namespace {
 // that the scoring launch holds about 2048 waves.
 struct IvfLayout {
   size_t cent, count, off, ids, centT, muL, assign, rank, tcount, pbest, total;
-  int64_t ntiles, stiles, groups, per_group;
+  int64_t ntiles, groups;
 };
 
 IvfLayout ivf_layout(int64_t BH, int64_t nb, int64_t nlist, int64_t d) {
   IvfLayout L;
   L.ntiles = (nb + kTile - 1) / kTile;
-  const int64_t gmax = (nlist + kAssignC - 1) / kAssignC;
-  L.stiles = (nb + 2 * kScoreTile - 1) / (2 * kScoreTile);
-  int64_t g = (2048 + L.stiles * BH - 1) / (L.stiles * BH);
-  L.groups = g < 1 ? 1 : (g > gmax ? gmax : g);
-  L.per_group = (nlist + L.groups - 1) / L.groups;
+  L.groups = ScoreSplit(nb, BH, nlist, nlist).groups;
   size_t o = 0;
   L.cent = o;   o += r256(size_t(BH) * nlist * d * 4);
   L.count = o;  o += r256(size_t(BH) * nlist * 4);
@@ -288,14 +284,12 @@ extern "C" int ssa_ivf_build(const float* mu, int64_t BH, int64_t nb, int64_t d,
   float* muL = reinterpret_cast<float*>(base + L.muL);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const dim3 gc((unsigned)nlist, (unsigned)BH), gt((unsigned)L.ntiles, (unsigned)BH);
-  const dim3 gs((unsigned)L.stiles, (unsigned)BH, (unsigned)L.groups);
+  const ssa::ScoreSplit split(nb, BH, nlist, nlist);
   ssa::ivf_init_kernel<<<gc, 64, 0, s>>>(mu, nb, d, nlist, cent);
   SSA_TRY(ssa::launch_status("ivf_init_kernel"));
   for (int64_t it = 0; it <= niter; ++it) {
     const bool last = it == niter;  // the last assignment only fills the lists
-    ssa::ivf_score_kernel<<<gs, ssa::kScoreTile, ssa::kAssignC * d * sizeof(double), s>>>(
-        mu, cent, nb, d, nlist, L.per_group, pbest);
-    SSA_TRY(ssa::launch_status("ivf_score_kernel"));
+    SSA_TRY(ssa::ivf_score(mu, cent, BH, nb, d, nlist, split, pbest, s));
     ssa::ivf_rank_kernel<<<gt, ssa::kTile, 0, s>>>(pbest, nb, nlist, L.ntiles, L.groups, assign,
                                                     rank, tcount);
     SSA_TRY(ssa::launch_status("ivf_rank_kernel"));

@@ -13,9 +13,8 @@ namespace {
 constexpr int kIvfMaxD = 256;      // head dim: a multiple of 32, at most this
 constexpr int kIvfCap = 2048;      // LDS keys per route pass (coarse keys, candidates, the union)
 constexpr int kIvfMaxSearch = kIvfCap / 2;
-constexpr int kAssignC = 16;       // centroids staged in LDS per assignment pass
 constexpr int kTile = 256;         // block means per rank / scatter workgroup
-constexpr int kScoreTile = 64;     // block means per scoring workgroup (one wave)
+constexpr int kScoreRows = 128;    // block means per scoring workgroup
 
 inline size_t r256(size_t x) { return (x + 255) & ~size_t(255); }
 
@@ -123,87 +122,144 @@ __device__ unsigned long long block_kth_largest(const unsigned long long* keys, 
 }
 
 // ---- build --------------------------------------------------------------------------------------
-// One wave per (tile of 128 block means, centroid group): the key of the best centroid of the
-// group for each block mean (largest inner product, ties to the lower centroid). Each lane owns
-// block means j and j + 64, so every staged centroid value (widened to fp64 once, when staged in
-// LDS, 2 per 16-byte read) feeds two fp64 chains with no conversion in the loop. Dynamic LDS:
-// kAssignC * d doubles.
-__global__ __launch_bounds__(kScoreTile) void ivf_score_kernel(
-    const float* __restrict__ mu, const float* __restrict__ cent, int64_t nb, int64_t d,
-    int64_t nlist, int64_t per_group, unsigned long long* __restrict__ pbest) {
-  extern __shared__ double scd[];  // d x kAssignC: element t of centroid c0 + c at t * kAssignC + c
-  const int tid = threadIdx.x;
-  const int64_t bh = blockIdx.y, tile = blockIdx.x, g = blockIdx.z;
-  int64_t j[2];
-  bool live[2];
-  const float* row[2];
+// A wave scores 32 block means (a workgroup of four: kScoreRows) against one group of `per_group`
+// 16-centroid tiles: pbest = the key of the group's best centroid for each mean (largest inner
+// product, ties to the lower centroid). v_mfma_f64_16x16x4_f64 (lane l supplies A[l%16][l/16] and
+// B[l/16][l%16]; accumulator r of lane l is C[4r + l/16][l%16]): A = the centroids, B = the means,
+// step s the dimensions 4 s .. 4 s + 3, which the unit adds in that order, one rounding each: the
+// bits of the fma chain in dimension order. d = 32 NC. A lane loads 16 bytes of a row at a time
+// (4 bytes a lane, one per step, fetched each line eight times: 16.2 us) and quarter_transpose
+// hands every lane the dimensions of its steps; the means stay in registers, the next tile's
+// centroids are loaded while this one's are multiplied, and nothing goes through LDS: as fma chains
+// over staged centroids a wave spent its time on the staging's bank conflicts and on four waits for
+// its rows. d 64: 8192 means, 90 centroids 20 -> 6.6 us (the matrix rate alone: 1.3); 8192 to 32,768
+// means, 181 centroids 23 -> 11.5 on average. What is left is the launch and one wait for the rows.
+typedef double ivf_f64x4 __attribute__((ext_vector_type(4)));
+
+// Element e of the lanes of quarter q (lane / 16) <-> element q of the lanes of quarter e.
+__device__ inline f32x4 quarter_transpose(const f32x4& x) {
+  unsigned int u[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) u[e] = __float_as_uint(x[e]);
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const auto r = __builtin_amdgcn_permlane32_swap(u[e], u[e + 2], false, false);
+    u[e] = r[0];
+    u[e + 2] = r[1];
+  }
+#pragma unroll
+  for (int e = 0; e < 4; e += 2) {
+    const auto r = __builtin_amdgcn_permlane16_swap(u[e], u[e + 1], false, false);
+    u[e] = r[0];
+    u[e + 1] = r[1];
+  }
+  return f32x4{__uint_as_float(u[0]), __uint_as_float(u[1]), __uint_as_float(u[2]),
+               __uint_as_float(u[3])};
+}
+
+template <int NC>
+__global__ __launch_bounds__(256) void ivf_score_kernel(
+    const float* __restrict__ mu, const float* __restrict__ cent, int64_t nb, int64_t nlist,
+    int64_t per_group, unsigned long long* __restrict__ pbest) {
+  constexpr int D = 32 * NC, NV = D / 16;  // 16-byte loads of a lane per row
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, col = lane & 15, kq = lane >> 4;
+  const int64_t bh = blockIdx.y, g = blockIdx.z;
+  const int64_t j0 = (int64_t)blockIdx.x * kScoreRows + 32 * w;
+  if (j0 >= nb) return;
+  f32x4 b[2][NV];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    j[h] = tile * 2 * kScoreTile + h * kScoreTile + tid;
-    live[h] = j[h] < nb;
-    row[h] = mu + (bh * nb + (live[h] ? j[h] : nb - 1)) * d;  // idle lanes read a valid row
+    const int64_t j = j0 + 16 * h + col < nb ? j0 + 16 * h + col : nb - 1;
+    const float* row = mu + (bh * nb + j) * D + 4 * kq;
+#pragma unroll
+    for (int v = 0; v < NV; ++v) b[h][v] = *reinterpret_cast<const f32x4*>(row + 16 * v);
   }
-  const float* cb = cent + bh * nlist * d;
-  const int64_t cbeg = g * per_group;
-  const int64_t cend = cbeg + per_group < nlist ? cbeg + per_group : nlist;
+  const float* cb = cent + bh * nlist * D + 4 * kq;
+  const int tiles = (int)((nlist + 15) / 16);
+  const int tbeg = (int)(g * per_group);
+  const int tend = tbeg + (int)per_group < tiles ? tbeg + (int)per_group : tiles;
+  auto load = [&](int tile, f32x4* a) {  // (rows past the last centroid re-read it: discarded)
+    const int64_t c = 16 * (int64_t)tile + col < nlist ? 16 * (int64_t)tile + col : nlist - 1;
+#pragma unroll
+    for (int v = 0; v < NV; ++v) a[v] = *reinterpret_cast<const f32x4*>(cb + c * D + 16 * v);
+  };
   unsigned long long best[2] = {0ull, 0ull};
-  for (int64_t c0 = cbeg; c0 < cend; c0 += kAssignC) {
-    const int cc = (int)(cend - c0 < kAssignC ? cend - c0 : kAssignC);
-    __syncthreads();
-    for (int e = tid; e < kAssignC * (int)d; e += kScoreTile) {
-      const int c = e / (int)d, t = e - c * (int)d;
-      scd[t * kAssignC + c] = c < cc ? (double)cb[(c0 + c) * d + t] : 0.0;
-    }
-    __syncthreads();
-    double acc[2][kAssignC];
+  f32x4 a[NV];
+  if (tbeg < tend) load(tbeg, a);
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+  for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int c = 0; c < kAssignC; ++c) acc[h][c] = 0.0;
-    for (int64_t t0 = 0; t0 < d; t0 += 16) {
-      float r[2][16];
+    for (int v = 0; v < NV; ++v) b[h][v] = quarter_transpose(b[h][v]);
+  for (int tile = tbeg; tile < tend; ++tile) {
+    f32x4 an[NV];
+    load(tile + 1 < tend ? tile + 1 : tile, an);
+    ivf_f64x4 acc[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
+    for (int v = 0; v < NV; ++v) {
+      const f32x4 at = quarter_transpose(a[v]);
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const float4 x = *reinterpret_cast<const float4*>(row[h] + t0 + 4 * u);
-          r[h][4 * u] = x.x;
-          r[h][4 * u + 1] = x.y;
-          r[h][4 * u + 2] = x.z;
-          r[h][4 * u + 3] = x.w;
-        }
+      for (int e = 0; e < 4; ++e)
 #pragma unroll
-      for (int t = 0; t < 16; ++t) {
-        const double2* s2 = reinterpret_cast<const double2*>(scd + (t0 + t) * kAssignC);
-        double cv[kAssignC];
-#pragma unroll
-        for (int q = 0; q < kAssignC / 2; ++q) {
-          const double2 x = s2[q];
-          cv[2 * q] = x.x;
-          cv[2 * q + 1] = x.y;
-        }
-        const double r0 = r[0][t], r1 = r[1][t];
-#pragma unroll
-        for (int c = 0; c < kAssignC; ++c) {
-          acc[0][c] = fma(r0, cv[c], acc[0][c]);
-          acc[1][c] = fma(r1, cv[c], acc[1][c]);
-        }
-      }
+        for (int h = 0; h < 2; ++h)
+          acc[h] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)at[e], (double)b[h][v][e], acc[h],
+                                                        0, 0, 0);
     }
 #pragma unroll
-    for (int c = 0; c < kAssignC; ++c) {
-      if (c < cc) {
+    for (int r = 0; r < 4; ++r) {
+      const int c = 16 * tile + 4 * r + kq;
+      if (c < nlist) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-          const unsigned long long k = ivf_key((float)acc[h][c], c0 + c);
+          const unsigned long long k = ivf_key((float)acc[h][r], c);
           best[h] = k > best[h] ? k : best[h];
         }
       }
     }
+#pragma unroll
+    for (int v = 0; v < NV; ++v) a[v] = an[v];
   }
 #pragma unroll
-  for (int h = 0; h < 2; ++h)
-    if (live[h]) pbest[(bh * gridDim.z + g) * nb + j[h]] = best[h];
+  for (int h = 0; h < 2; ++h) {
+#pragma unroll
+    for (int o = 16; o <= 32; o <<= 1) {
+      const unsigned long long k = __shfl_xor(best[h], o);
+      best[h] = k > best[h] ? k : best[h];
+    }
+    const int64_t j = j0 + 16 * h + col;
+    if (kq == 0 && j < nb) pbest[(bh * gridDim.z + g) * nb + j] = best[h];
+  }
+}
+
+// How ivf_score_kernel's launch splits the centroids: as many groups as give it about 2048 waves
+// (two per SIMD), at most `gmax` and at most one per 16 centroids.
+struct ScoreSplit {
+  int64_t wgs, groups, per_group;  // workgroups over the means; groups of per_group tiles
+  ScoreSplit(int64_t m, int64_t heads, int64_t nlist, int64_t gmax) {
+    const int64_t tiles = (nlist + 15) / 16;
+    wgs = (m + kScoreRows - 1) / kScoreRows;
+    int64_t g = (2048 + 4 * wgs * heads - 1) / (4 * wgs * heads);
+    g = g > tiles ? tiles : g;
+    g = g > gmax ? gmax : g;
+    g = g < 1 ? 1 : g;
+    per_group = (tiles + g - 1) / g;
+    groups = (tiles + per_group - 1) / per_group;
+  }
+};
+
+inline int ivf_score(const float* mu, const float* cent, int64_t heads, int64_t m, int64_t d,
+                     int64_t nlist, const ScoreSplit& sp, unsigned long long* pbest,
+                     hipStream_t s) {
+  const dim3 grid((unsigned)sp.wgs, (unsigned)heads, (unsigned)sp.groups);
+#define SSA_SCORE(NC)                                                                        \
+  case NC:                                                                                   \
+    ivf_score_kernel<NC><<<grid, 256, 0, s>>>(mu, cent, m, nlist, sp.per_group, pbest);      \
+    break
+  switch (d / 32) {  // d: a multiple of 32, at most kIvfMaxD
+    SSA_SCORE(1); SSA_SCORE(2); SSA_SCORE(3); SSA_SCORE(4);
+    SSA_SCORE(5); SSA_SCORE(6); SSA_SCORE(7); SSA_SCORE(8);
+  }
+#undef SSA_SCORE
+  return launch_status("ivf_score_kernel");
 }
 
 // The rank of this thread's centroid a (-1: none) among the threads before it of a 256-thread tile

@@ -121,6 +121,23 @@ def test_ivf_lists_match_oracle(cuda, nb, nlist):
             assert ids[h, off[h, c]:off[h, c + 1]].tolist() == lists[c].tolist(), (h, c)
 
 
+# list scoring (16-centroid tiles, 32 means a wave) and updates (runs of 64 members): every head dim
+# the kernels are built for, remainders of each tile, lists of one member, of a run and of several
+@pytest.mark.parametrize("nb,nlist,d", [(1100, 2, 64), (500, 33, 96), (97, 16, 128), (130, 5, 160),
+                                        (1, 1, 192), (129, 128, 224), (700, 3, 256)])
+def test_ivf_scores_and_updates_match_oracle(cuda, nb, nlist, d):
+    from ssa_amd import ivf_kernel as I
+    rng = np.random.default_rng(d)
+    mu = rng.standard_normal((2, nb, d)).astype(np.float32)
+    ix = I.build_ivf(torch.from_numpy(mu).to(cuda), nlist=nlist, niter=3)
+    off, ids = ix.list_offsets.cpu().numpy(), ix.list_ids.cpu().numpy()
+    for h in range(2):
+        cent, lists = O.ivf_build(mu[h], nlist, 3)
+        assert (ix.centroids[h].cpu().numpy() == cent).all()
+        for c in range(nlist):
+            assert ids[h, off[h, c]:off[h, c + 1]].tolist() == lists[c].tolist(), (h, c)
+
+
 # masked attention: one block per key tile and several, a block of two tiles, a length that
 # ends inside a wave's rows, more than the 64 tiles of a mask round (4100 tokens), grouped heads
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
