@@ -104,8 +104,9 @@ constexpr int kStreamRun = 4 * kIvfCap;  // candidates of a run once a threshold
 // below the threshold that kept them (K keys above it already) cannot enter the K largest and is
 // dropped on arrival, so later batches fill the buffer slowly. buf[0..nk0) may hold up to K keys
 // of earlier candidates (nonzero, visible to the workgroup), ranked with the M new ones. Returns
-// how many are kept (in buf[0..), any order). 256 threads.
-template <typename F>
+// how many are kept (in buf[0..), any order). 256 threads, U candidates of each in flight (past
+// U = 2 keyof is a few loads, without a branch, and the last candidates are read again).
+template <int U, typename F>
 __device__ int stream_top(unsigned long long* buf, int64_t M, int K, F keyof, unsigned int* hist,
                           unsigned int* shv, int* ws, int nk0 = 0) {
   int nk = nk0;
@@ -120,18 +121,18 @@ __device__ int stream_top(unsigned long long* buf, int64_t M, int K, F keyof, un
       if (batch > kStreamRun) batch = kStreamRun;
       if (threadIdx.x == 0) ws[0] = 0;
       __syncthreads();
-      for (int e = threadIdx.x; e < batch; e += 512) {
-        const bool two = e + 256 < batch;
-        const unsigned long long k0 = keyof(m0 + e);
-        const unsigned long long k1 = two ? keyof(m0 + e + 256) : 0ull;
+      for (int e = threadIdx.x; e < batch; e += 256 * U) {
+        unsigned long long k[U];
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const unsigned long long k = u ? k1 : k0;
-          if (k >= floor_key) {
+        for (int u = 0; u < U; ++u)
+          k[u] = U > 2 || e + 256 * u < batch
+                     ? keyof(m0 + (e + 256 * u < batch ? e + 256 * u : batch - 1)) : 0ull;
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (e + 256 * u < batch && k[u] >= floor_key) {
             const int at = atomicAdd(&ws[0], 1);
-            if (at < room) buf[nk + at] = k;
+            if (at < room) buf[nk + at] = k[u];
           }
-        }
       }
       __syncthreads();
       const int got = ws[0];
@@ -143,12 +144,15 @@ __device__ int stream_top(unsigned long long* buf, int64_t M, int K, F keyof, un
     }
     if (!done) {
       batch = M - m0 < room ? M - m0 : room;
-      for (int e = threadIdx.x; e < batch; e += 512) {  // two candidates per thread per pass
-        const bool two = e + 256 < batch;
-        const unsigned long long k0 = keyof(m0 + e);
-        const unsigned long long k1 = two ? keyof(m0 + e + 256) : 0ull;
-        buf[nk + e] = k0 >= floor_key ? k0 : 0ull;
-        if (two) buf[nk + e + 256] = k1 >= floor_key ? k1 : 0ull;
+      for (int e = threadIdx.x; e < batch; e += 256 * U) {
+        unsigned long long k[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          k[u] = U > 2 || e + 256 * u < batch
+                     ? keyof(m0 + (e + 256 * u < batch ? e + 256 * u : batch - 1)) : 0ull;
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (e + 256 * u < batch) buf[nk + e + 256 * u] = k[u] >= floor_key ? k[u] : 0ull;
       }
       __syncthreads();
       nk = block_compact<unsigned long long>(buf, nk + (int)batch, buf, ws,
@@ -662,7 +666,7 @@ struct CccRouteLds {
 // SCORED: the scores against the staged means, the flat committed means and the outlier keys were
 // written by ccc_score_kernel; the members of probed lists are always scored here.
 template <bool SCORED>
-__global__ __launch_bounds__(256, 4) void ccc_route_kernel(CccRouteArgs a) {
+__global__ __launch_bounds__(256, SCORED ? 4 : 3) void ccc_route_kernel(CccRouteArgs a) {
   __shared__ unsigned long long buf[kIvfCap];     // streamed keys, then the merged candidates
   __shared__ __align__(16) float qs[kIvfMaxD];
   // the rest by this call's sizes (CccRouteLds)
@@ -695,18 +699,23 @@ __global__ __launch_bounds__(256, 4) void ccc_route_kernel(CccRouteArgs a) {
   }
   const float* means = a.means;
   const int64_t spb = a.spb, committed = a.committed;
+  const unsigned int sb = (unsigned int)spb;  // (sub-mean indices are below 2^32)
+  // Candidates a thread has in flight where one is a load: with 2, behind a 64-bit division each to
+  // find the parent, a chunk of 1024 query blocks (12,288 staged sub-means, 181 cells) took 182 us,
+  // now 162; the division is a length of the walk (staged) or a compare (parents) instead.
+  constexpr int UF = SCORED ? 8 : 2;
   const float* score = SCORED ? a.score + i * a.sld : nullptr;
 
   // the staged sub-means (exhaustive, causally masked: parent strictly before the query block)
   const int64_t ns = a.n_sub - committed;
   const int ks = (int)(a.ks < ns ? a.ks : ns);
+  const int64_t past = qblk * spb - committed < ns ? qblk * spb - committed : ns;
   int nst = 0;
-  if (ks > 0) {
-    nst = stream_top(
-        buf, ns, ks,
+  if (ks > 0 && past > 0) {
+    nst = stream_top<UF>(
+        buf, past, ks,
         [&](int64_t m) -> unsigned long long {
           const int64_t j = committed + m;
-          if (j / spb >= qblk) return 0ull;
           return ivf_key(SCORED ? score[m] : dot_row(qs, means + j * d, d), j);
         },
         hist, shv, ws);
@@ -732,7 +741,7 @@ __global__ __launch_bounds__(256, 4) void ccc_route_kernel(CccRouteArgs a) {
     unsigned long long Tc = 0ull;
     if (committed > 0 && kc > 0) {
       if (!a.has_index) {
-        ncm = stream_top(
+        ncm = stream_top<UF>(
             buf, committed, (int)kc,
             [&](int64_t m) -> unsigned long long {
               return ivf_key(SCORED ? score[a.soff_com + m] : dot_row(qs, means + m * d, d), m);
@@ -781,7 +790,7 @@ __global__ __launch_bounds__(256, 4) void ccc_route_kernel(CccRouteArgs a) {
         mtot += M;
         for (int e = tid; e < ncarry; e += 256) buf[e] = carry[e];
         __syncthreads();
-        ncm = stream_top(
+        ncm = stream_top<2>(
             buf, M, carry != nullptr ? (int)a.kkeep : (int)kc,
             [&](int64_t m) -> unsigned long long {
               int lo = 0, hi = np - 1;
@@ -822,10 +831,10 @@ __global__ __launch_bounds__(256, 4) void ccc_route_kernel(CccRouteArgs a) {
       drop[u] = false;
       if (e < n) {
         const unsigned long long v = buf[e];
-        const int64_t p = ivf_key_index(v) / spb;
+        const unsigned int first = (unsigned int)ivf_key_index(v) / sb * sb;  // of its parent
         for (int f = 0; f < n; ++f) {
           const unsigned long long y = buf[f];
-          if (y > v && ivf_key_index(y) / spb == p) {
+          if (y > v && (unsigned int)ivf_key_index(y) - first < sb) {
             drop[u] = true;
             break;
           }
@@ -848,7 +857,7 @@ __global__ __launch_bounds__(256, 4) void ccc_route_kernel(CccRouteArgs a) {
                                           [T](unsigned long long k) { return k >= T; });
       }
       tau = key_score(block_min_key(buf, K, kslot));
-      for (int e = tid; e < K; e += 256) lst[e] = (int)(ivf_key_index(buf[e]) / spb);
+      for (int e = tid; e < K; e += 256) lst[e] = (int)((unsigned int)ivf_key_index(buf[e]) / sb);
       __syncthreads();
     }
 
@@ -858,12 +867,12 @@ __global__ __launch_bounds__(256, 4) void ccc_route_kernel(CccRouteArgs a) {
     if (cap > 0) {
       const float* ov = a.ovec;
       const int64_t* op = a.opar;
-      nop = stream_top(
+      nop = stream_top<UF>(
           buf, a.n_out, cap,
           [&](int64_t r) -> unsigned long long {
-            if (op[r] >= qblk) return 0ull;
+            if (!SCORED && op[r] >= qblk) return 0ull;
             const float s = SCORED ? score[a.soff_out + r] : dot_row(qs, ov + r * d, d);
-            return s > tau ? ivf_key(s, r) : 0ull;
+            return s > tau && (!SCORED || op[r] < qblk) ? ivf_key(s, r) : 0ull;
           },
           hist, shv, ws);
       for (int e = tid; e < nop; e += 256) lst[K + e] = (int)op[ivf_key_index(buf[e])];
@@ -1229,7 +1238,7 @@ extern "C" int ssa_ccc_route(const float* qr, int64_t nbq, int64_t qb_start, int
   a.means = means;
   a.committed = committed;
   a.n_sub = n_sub;
-  a.spb = spb;
+  a.spb = spb < (int64_t(1) << 31) ? spb : int64_t(1) << 31;  // (no index reaches 2^31: the same parents)
   a.ovec = out_vec;
   a.opar = out_parent;
   a.n_out = n_out;

@@ -105,6 +105,27 @@ def test_cascade_route_scores_match_oracle(cuda, monkeypatch, d, blocks, nbq, ri
         assert ki[i, :rn[i]].tolist() == rl[i], i
 
 
+# the same for query blocks at and before the staged means' first block (none, one or two are past)
+@pytest.mark.parametrize("limit", [None, 0])
+def test_cascade_route_before_the_staged_means(cuda, monkeypatch, limit):
+    from ssa_amd import cascade_router as C
+    if limit is not None:
+        monkeypatch.setattr(C, "SCORE_WORKSPACE_LIMIT", limit)
+    rng = np.random.default_rng(5)
+    k = rng.standard_normal((24 * 128, 64)).astype(np.float16)
+    q = rng.standard_normal((8 * 128, 64)).astype(np.float16)
+    got, ref = C.CausalCascade(64, search_k=48), O.CascadeOracle(64, search_k=48)
+    for a, b in ((0, 16), (16, 24)):
+        got.append(torch.from_numpy(k[a * 128:b * 128]).to(cuda))
+        ref.append(k[a * 128:b * 128].astype(np.float32))
+    for first in (14, 16):  # (staged: blocks 16 .. 23)
+        kn, ki, _, _ = got.route(torch.from_numpy(q).to(cuda), first * 128)
+        rn, rl, _, _ = ref.route(q.astype(np.float32), first * 128)
+        assert (kn.cpu().numpy() == rn).all()
+        for i in range(8):
+            assert ki[i, :rn[i]].tolist() == rl[i], (first, i)
+
+
 # list building: one wave, one tile and several, with remainders; one list, a list per mean, the most
 @pytest.mark.parametrize("nb,nlist", [(33, 1), (64, 64), (256, 17), (257, 257), (1000, 300),
                                       (2300, 2048)])
