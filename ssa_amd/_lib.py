@@ -166,8 +166,9 @@ def ptr(t: torch.Tensor | None) -> int | None:
 
 
 def stream_of(t: torch.Tensor) -> int:
-    """The current HIP stream of t's device as a raw handle."""
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """The current HIP stream of t's device as a raw handle (without a torch.cuda.Stream around it,
+    which cost as much as the launch)."""
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 def i64_array(values) -> ctypes.Array:

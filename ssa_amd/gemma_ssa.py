@@ -255,8 +255,11 @@ def _query_path_summaries(module, key, q_len, pos0, with_m3, block):
     if st is None or st["sig"] != sig or pos0 != st["kv_len"] or kv_len != st["kv_len"] + q_len:
         st = {"sig": sig, "kv_len": 0, "nc": 0, "mu": None, "var": None, "m3": None}
         _DECODE[lk] = st
-    if st["mu"] is None or st["mu"].shape[2] < nb:  # capacity doubles, contents kept
-        cap = max(nb, 2 * (0 if st["mu"] is None else st["mu"].shape[2]), 64)
+    if st["mu"] is None or st["mu"].shape[2] < nb:
+        # Contents kept. Exactly nb entries, which the router reads as they are: with spare capacity
+        # every step copied mu and var to hand it contiguous ones (16 of 41 launches over 8 steps),
+        # now once per block of tokens. One head's views are contiguous as they are: capacity doubles.
+        cap = nb if b * hkv > 1 else max(nb, 2 * (0 if st["mu"] is None else st["mu"].shape[2]), 64)
         for name in ("mu", "var", "m3"):
             if name == "m3" and not with_m3:
                 continue
