@@ -344,40 +344,40 @@ __global__ __launch_bounds__(256) void ivf_tile_prefix_kernel(int32_t* __restric
   if (threadIdx.x == 0) count[bh * nlist + c] = running;
 }
 
-// One workgroup per head: off[c] = the members of the centroids before c, off[nlist] = all.
-__global__ __launch_bounds__(256) void ivf_offsets_kernel(const int32_t* __restrict__ count,
-                                                           int64_t nlist,
-                                                           int32_t* __restrict__ off) {
-  __shared__ int ws[4];
-  const int64_t bh = blockIdx.x;
-  const int tid = threadIdx.x;
-  int running = 0;
-  for (int64_t c0 = 0; c0 < nlist; c0 += 256) {
-    const int64_t c = c0 + tid;
-    const int v = c < nlist ? count[bh * nlist + c] : 0;
-    int tot;
-    const int ex = ivf_block_scan(v, ws, &tot);
-    if (c < nlist) off[bh * (nlist + 1) + c] = running + ex;
-    running += tot;
-  }
-  if (tid == 0) off[bh * (nlist + 1) + nlist] = running;
-}
-
 // One thread per block mean: its slot in ids = offset of its list + members of the list in
 // earlier tiles (tbase, the prefix of ivf_tile_prefix_kernel) + its rank in its tile. With muL set
 // (the last assignment), the mean is also copied to its list's transposed storage: element t of
-// member k of list p at d * off[p] + t * size[p] + k.
+// member k of list p at d * off[p] + t * size[p] + k. Every workgroup adds up the list sizes for
+// itself (nlist <= kIvfCap) and the first one of a head writes off[c] = the members of the centroids
+// before c, off[nlist] = all: a launch of its own for that took 2.5 us and a gap beside this kernel's
+// 4.8, now 5.5 (1M-token IVF prefill 906 -> 881 us).
 __global__ __launch_bounds__(256) void ivf_scatter_kernel(
     const int32_t* __restrict__ assign, const int32_t* __restrict__ rank,
     const int32_t* __restrict__ tbase, int64_t nb, int64_t nlist, int64_t ntiles,
-    const int32_t* __restrict__ count, const int32_t* __restrict__ off, int32_t* __restrict__ ids,
+    const int32_t* __restrict__ count, int32_t* __restrict__ off, int32_t* __restrict__ ids,
     const float* __restrict__ mu, int64_t d, float* __restrict__ muL) {
+  __shared__ int start[kIvfCap];
+  __shared__ int ws[4];
   const int64_t bh = blockIdx.y, tile = blockIdx.x;
   const int64_t j = tile * kTile + threadIdx.x;
+  const int a = j < nb ? assign[bh * nb + j] : 0;
+  const int r = j < nb ? tbase[(bh * ntiles + tile) * nlist + a] + rank[bh * nb + j] : 0;
+  int running = 0;
+  for (int64_t c0 = 0; c0 < nlist; c0 += 256) {
+    const int64_t c = c0 + threadIdx.x;
+    const int v = c < nlist ? count[bh * nlist + c] : 0;
+    int tot;
+    const int at = running + ivf_block_scan(v, ws, &tot);
+    if (c < nlist) {
+      start[c] = at;
+      if (tile == 0) off[bh * (nlist + 1) + c] = at;
+    }
+    running += tot;
+  }
+  if (tile == 0 && threadIdx.x == 0) off[bh * (nlist + 1) + nlist] = running;
+  __syncthreads();
   if (j >= nb) return;
-  const int a = assign[bh * nb + j];
-  const int o = off[bh * (nlist + 1) + a];
-  const int pos = o + tbase[(bh * ntiles + tile) * nlist + a] + rank[bh * nb + j];
+  const int o = start[a], pos = o + r;
   ids[bh * nb + pos] = (int32_t)j;
   if (muL != nullptr) {
     const int64_t L = count[bh * nlist + a];
@@ -396,8 +396,6 @@ inline int ivf_lists(const int32_t* assign, const int32_t* rank, int32_t* tcount
   ivf_tile_prefix_kernel<<<dim3((unsigned)nlist, (unsigned)BH), 256, 0, s>>>(tcount, ntiles,
                                                                              nlist, count, nullptr);
   SSA_TRY(launch_status("ivf_tile_prefix_kernel"));
-  ivf_offsets_kernel<<<(unsigned)BH, 256, 0, s>>>(count, nlist, off);
-  SSA_TRY(launch_status("ivf_offsets_kernel"));
   ivf_scatter_kernel<<<dim3((unsigned)ntiles, (unsigned)BH), 256, 0, s>>>(
       assign, rank, tcount, nb, nlist, ntiles, count, off, ids, mu, d, muL);
   return launch_status("ivf_scatter_kernel");
