@@ -458,10 +458,11 @@ __device__ inline void block_partial_128(const DecodeParams& p, float* part, flo
     }
     const float s = (sc[0] + lane_xor(sc[0], 1)) * p.scale_log2;  // key k0 + kg + 4 (ch >> 1)
     const int mine = k0 + kg + 4 * (ch >> 1);
-    const float mnew = fmaxf(m, wave_max(mine < nk ? s : -INFINITY));  // (key k0 is in range)
-    const float alpha = exp2f(m - mnew);
+    const float mnew = fmaxf(m, wave_max(mine < nk ? s : -INFINITY));
+    const float mref = mnew == -INFINITY ? 0.0f : mnew;  // (no key of a finite score so far)
+    const float alpha = exp2f(m - mref);
     m = mnew;
-    const float pk = mine < nk ? exp2f(s - mnew) : 0.0f;
+    const float pk = mine < nk ? exp2f(s - mref) : 0.0f;
     wave_lds_sync();  // the previous 32 keys' weights have been read
     if ((ch & 1) == 0) ps[kg + 4 * (ch >> 1)] = pk;
     l = l * alpha + ((ch & 1) == 0 ? pk : 0.0f);

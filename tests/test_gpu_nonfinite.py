@@ -1,0 +1,63 @@
+"""GPU kernels on inputs with infinities: a value that takes no part in a row (a weight of zero, a
+key or a row past the end) leaves no trace in it. Against the CPU oracle (float64)."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import ssa_oracle as O
+from ssa_amd import workloads as WL
+
+pytestmark = pytest.mark.gpu
+INF = float("inf")
+
+
+def np_of(t):
+    return t.detach().float().cpu().numpy()
+
+
+def same(got, ref, tol):
+    """Equal infinities, no NaN where the reference has none, finite values within tol."""
+    f = np.isfinite(ref)
+    assert (np.isfinite(got) == f).all()
+    assert (got[~f] == ref[~f]).all()
+    assert np.abs(got[f] - ref[f]).max() < tol
+
+
+def decode_all_blocks(cuda, dtype, d, block, n, poison, steps=2):
+    """Steps of a decoder that selects every block of an n-token cache, and the oracle's rows.
+    poison(k, v): sets values of the n + steps tokens before they are used (CPU arrays)."""
+    from ssa_amd.ivf_decode import RoutedDecoder
+    rng = np.random.default_rng(n + d + block)
+    hq, hkv = 4, 2
+    k, v = (WL.round_to(rng.standard_normal((1, hkv, n + steps, d)).astype(np.float32), dtype)
+            for _ in range(2))
+    q = WL.round_to(rng.standard_normal((steps, 1, hq, d)).astype(np.float32), dtype)
+    q[..., 0] = np.abs(q[..., 0]) + 0.5
+    nb = -(-(n + steps) // block)
+    dec = RoutedDecoder(1, hq, hkv, d, n + steps, block=block, top_c=nb, local=1, dtype=dtype,
+                        device=cuda)
+    kt, vt, qt = (WL.to_device(a, dtype, cuda) for a in (k, v, q))
+    dec.prefill(kt[:, :, :n], vt[:, :, :n])  # (the routing summaries stay finite)
+    poison(k, v)
+    kt, vt = (WL.to_device(a, dtype, cuda) for a in (k, v))
+    dec.kcache[:, :, :n], dec.vcache[:, :, :n] = kt[:, :, :n], vt[:, :, :n]
+    for t in range(steps):
+        out = np_of(dec.step(qt[t], kt[:, :, n + t], vt[:, :, n + t]))
+        sel = list(range((n + t) // block + 1))
+        for h in range(hq):
+            assert dec.kv_idx[0, h, :int(dec.kv_num[0, h])].tolist() == sel
+            ref = O.decode_attend(q[t][0, h], k[0, h // 2], v[0, h // 2], sel, n + t, block)
+            yield out[0, h], ref
+
+
+# the first 32 keys of a half block score -inf (block 128), a whole half does (block 64)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("block", [64, 128])
+def test_decode_step_keys_of_minus_infinity(cuda, dtype, block):
+    n = 3 * block + 5 * block // 8
+
+    def poison(k, v):
+        for half in (block, 3 * block):  # a half of a complete block, and of the own one
+            k[:, :, half:half + 32, 0] = -INF
+    for got, ref in decode_all_blocks(cuda, dtype, 128, block, n, poison):
+        same(got, ref, 2e-2)
