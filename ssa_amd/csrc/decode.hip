@@ -469,6 +469,10 @@ __device__ inline void block_partial_128(const DecodeParams& p, float* part, flo
     wave_lds_sync();
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[e] *= alpha;
+    if (nk - k0 < 4 * T)  // the last key read again: zeros (its infinities times weight 0 are NaN)
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+        if (k0 + kg + 4 * t >= nk) vx[t] = u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
     for (int t = 0; t < T; ++t) {
       float x[8];

@@ -61,3 +61,17 @@ def test_decode_step_keys_of_minus_infinity(cuda, dtype, block):
             k[:, :, half:half + 32, 0] = -INF
     for got, ref in decode_all_blocks(cuda, dtype, 128, block, n, poison):
         same(got, ref, 2e-2)
+
+
+# the last key of a part whose length fills no 32-key load: whole halves of 8, 16 and 32 keys, and
+# the whole block
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d,block", [(128, 16), (128, 32), (128, 64), (64, 32)])
+def test_decode_step_value_of_infinity_last_in_its_part(cuda, dtype, d, block):
+    n = 10 * block + block // 4
+
+    def poison(k, v):
+        v[:, :, block + block // 2 - 1, 7] = INF
+        v[:, :, 2 * block - 1, 9] = -INF
+    for got, ref in decode_all_blocks(cuda, dtype, d, block, n, poison):
+        same(got, ref, 2e-2)
