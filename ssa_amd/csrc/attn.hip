@@ -403,7 +403,7 @@ __global__ __launch_bounds__(NW * 64, 2) void sparse_attn_f32_kernel(AttnParams 
       }
     }
   };
-  // rows past the end re-read row n - 1 (their keys are masked)
+  // rows past the end re-read row n - 1 (their keys are masked, their values cleared)
   auto load_k = [&](int key0, f32x4* f) {
     int kr = key0 + col;
     if (kr > n32 - 1) kr = n32 - 1;
@@ -479,6 +479,10 @@ __global__ __launch_bounds__(NW * 64, 2) void sparse_attn_f32_kernel(AttnParams 
         l_part[c] += s[c][r];
       }
     }
+    if (key0 + 15 >= n32)  // row n - 1 read again: zeros (its infinities times weight 0 are NaN)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (key0 + 4 * quarter + r >= n32) vf[r] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int r = 0; r < 4; ++r)
 #pragma unroll

@@ -75,3 +75,32 @@ def test_decode_step_value_of_infinity_last_in_its_part(cuda, dtype, d, block):
         v[:, :, 2 * block - 1, 9] = -INF
     for got, ref in decode_all_blocks(cuda, dtype, d, block, n, poison):
         same(got, ref, 2e-2)
+
+
+# an infinite value in the last row of a length that fills no tile: rows that attend it are infinite
+@pytest.mark.parametrize("dtype,d,hq,hkv,n,block", [(torch.float32, 64, 2, 1, 700, 64),
+                                                    (torch.float32, 64, 8, 2, 2075, 128),
+                                                    (torch.bfloat16, 128, 2, 1, 300, 64)])
+def test_prefill_value_of_infinity_in_the_last_row(cuda, dtype, d, hq, hkv, n, block):
+    from ssa_amd import ssa_kernel as K
+    rng = np.random.default_rng(n)
+    q, k, v = (WL.round_to(rng.standard_normal((1, h, n, d)).astype(np.float32), dtype)
+               for h in (hq, hkv, hkv))
+    v[:, :, n - 1, 3], v[:, :, n - 1, 5] = INF, -INF
+    nb = -(-n // block)
+    num = np.minimum(np.arange(nb) + 1, 3)
+    idx = np.clip(np.arange(nb)[:, None] - num[:, None] + 1 + np.arange(3), 0, nb - 1)
+    num, idx = (np.broadcast_to(a.astype(np.int32), (1, hq, *a.shape)).copy() for a in (num, idx))
+    out = np_of(K.sparse_attention(*(WL.to_device(a, dtype, cuda) for a in (q, k, v)),
+                                   torch.from_numpy(num).to(cuda), torch.from_numpy(idx).to(cuda),
+                                   block))
+    finite = v.copy()
+    finite[:, :, n - 1, 3] = finite[:, :, n - 1, 5] = 0.0
+    ref = O.sparse_attention(q, k, finite, num, idx, block)
+    ref[:, :, n - 1, 3], ref[:, :, n - 1, 5] = INF, -INF
+    # (head dims without the infinity everywhere, all head dims in the last row; rows before it
+    # share a tile with the infinity at weight 0)
+    rest = [e for e in range(d) if e not in (3, 5)]
+    tol = 1e-5 if dtype == torch.float32 else 2e-2
+    same(out[..., rest], ref[..., rest], tol)
+    same(out[:, :, n - 1], ref[:, :, n - 1], tol)
