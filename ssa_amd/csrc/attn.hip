@@ -1268,11 +1268,10 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) void sparse_attn_wide16_k
     }
 #pragma unroll
     for (int j = 0; j < LPW; ++j) {
-      const int r = j * NW + w;
-      int kr = key0 + r;
-      if (kr > n32 - 1) kr = n32 - 1;
-      __builtin_amdgcn_global_load_lds(vbase + (int64_t)kr * p.vsn + ((lane ^ (2 * vswz(r))) * 8),
-                                       vdst + r * 1024, 16, 0, 0);
+      const int r = j * NW + w, kr = key0 + r;
+      const unsigned short* vr =  // ragged tail: zeros (a masked key's infinities times 0 are NaN)
+          kr < n32 ? vbase + (int64_t)kr * p.vsn : reinterpret_cast<const unsigned short*>(kZeroRow);
+      __builtin_amdgcn_global_load_lds(vr + ((lane ^ (2 * vswz(r))) * 8), vdst + r * 1024, 16, 0, 0);
     }
   };
 

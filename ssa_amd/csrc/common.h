@@ -115,6 +115,10 @@ __device__ inline void dma_barrier() {
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
+// The row that LDS DMA of a row past the last one reads: its weight is zero, but zero times an
+// infinity in a real row read twice would be NaN (1 KB: a 16-bit row of head dim 512).
+__device__ const u32x4 kZeroRow[64] = {};
+
 // Transposing LDS read (ds_read_b64_tr_b16): of the 16 lanes of a group, lane l gives the address
 // of four 16-bit values (its 8 bytes) and receives value l & 3 of lanes 4 j + (l >> 2), j = 0..3:
 // with lane l at row l >> 2, columns 4 (l & 3).. of a 4 x 16 block, column l of the block.

@@ -80,7 +80,10 @@ def test_decode_step_value_of_infinity_last_in_its_part(cuda, dtype, d, block):
 # an infinite value in the last row of a length that fills no tile: rows that attend it are infinite
 @pytest.mark.parametrize("dtype,d,hq,hkv,n,block", [(torch.float32, 64, 2, 1, 700, 64),
                                                     (torch.float32, 64, 8, 2, 2075, 128),
-                                                    (torch.bfloat16, 128, 2, 1, 300, 64)])
+                                                    (torch.bfloat16, 128, 2, 1, 300, 64),
+                                                    (torch.float16, 512, 16, 4, 797, 128),
+                                                    (torch.bfloat16, 512, 24, 8, 1043, 256),
+                                                    (torch.bfloat16, 512, 48, 8, 261, 64)])
 def test_prefill_value_of_infinity_in_the_last_row(cuda, dtype, d, hq, hkv, n, block):
     from ssa_amd import ssa_kernel as K
     rng = np.random.default_rng(n)
