@@ -257,14 +257,16 @@ __device__ inline void issue_pair32(const char* x, int64_t xs, const char* y, in
                                     int lane) {
   const float* xb = reinterpret_cast<const float*>(x);
   const float* yb = reinterpret_cast<const float*>(y);
+  const float* zero = reinterpret_cast<const float*>(kZeroRow);
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int r = (4 * j + w) * 4 + (lane >> 4);
-    const int64_t row = r0 + r < nrows ? r0 + r : nrows - 1;  // past the end: masked entries
+    const int64_t row = r0 + r;
     const int col = ((lane & 15) ^ (r & 15)) * 4;
-    __builtin_amdgcn_global_load_lds(xb + row * xs + col, st + (4 * j + w) * 1024, 16, 0, 0);
-    __builtin_amdgcn_global_load_lds(yb + row * ys + col, st + kPairTile32 + (4 * j + w) * 1024,
-                                     16, 0, 0);
+    const float* xr = row < nrows ? xb + row * xs : zero;  // past the end: masked entries
+    const float* yr = row < nrows ? yb + row * ys : zero;
+    __builtin_amdgcn_global_load_lds(xr + col, st + (4 * j + w) * 1024, 16, 0, 0);
+    __builtin_amdgcn_global_load_lds(yr + col, st + kPairTile32 + (4 * j + w) * 1024, 16, 0, 0);
   }
 }
 
@@ -657,8 +659,8 @@ __global__ __launch_bounds__(256, 2) void swap_dkdv_kernel(SwapArgs a) {
       if (at.qt < a.nqt) {
         at.mw = kvalid ? a.masks[(bh * a.nqt + at.qt) * a.nb + ck] : 0ull;
         const int64_t row = at.qt * 64 + lane;
-        if (tid < 128)  // (rows past the end belong to no list: any finite value will do)
-          at.ld = (tid < 64 ? a.lse : a.delta)[bh * a.n + (row < a.n ? row : a.n - 1)];
+        if (tid < 128)  // (rows past the end belong to no list, but an infinity would be NaN)
+          at.ld = row < a.n ? (tid < 64 ? a.lse : a.delta)[bh * a.n + row] : 0.0f;
         break;
       }
     }
@@ -781,19 +783,22 @@ constexpr int kPairTile = 64 * 128;
 __device__ inline int pair_swz(int r) { return ((r & 2) << 1) | ((r >> 2) & 3); }
 
 // Issues this wave's share of rows [r0, r0 + 64) of x and y (row strides in elements; rows past the
-// last one re-read it: their entries are masked) into st and st + kPairTile. 256 threads.
+// last one are zeros: their entries are masked, and 0 times an infinity of a real row read twice
+// would be NaN) into st and st + kPairTile. 256 threads.
 __device__ inline void issue_pair(const char* x, int64_t xs, const char* y, int64_t ys, int64_t r0,
                                   int64_t nrows, unsigned char* st, int w, int lane) {
   const unsigned short* xb = reinterpret_cast<const unsigned short*>(x);
   const unsigned short* yb = reinterpret_cast<const unsigned short*>(y);
+  const unsigned short* zero = reinterpret_cast<const unsigned short*>(kZeroRow);
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     const int r = (4 * j + w) * 8 + (lane >> 3);
-    const int64_t row = r0 + r < nrows ? r0 + r : nrows - 1;
+    const int64_t row = r0 + r;
     const int col = ((lane & 7) ^ pair_swz(r)) * 8;
-    __builtin_amdgcn_global_load_lds(xb + row * xs + col, st + (4 * j + w) * 1024, 16, 0, 0);
-    __builtin_amdgcn_global_load_lds(yb + row * ys + col, st + kPairTile + (4 * j + w) * 1024, 16,
-                                     0, 0);
+    const unsigned short* xr = row < nrows ? xb + row * xs : zero;
+    const unsigned short* yr = row < nrows ? yb + row * ys : zero;
+    __builtin_amdgcn_global_load_lds(xr + col, st + (4 * j + w) * 1024, 16, 0, 0);
+    __builtin_amdgcn_global_load_lds(yr + col, st + kPairTile + (4 * j + w) * 1024, 16, 0, 0);
   }
 }
 
@@ -1157,8 +1162,8 @@ __global__ __launch_bounds__(256, 2) void swap_dkdv16_kernel(SwapArgs a) {
       if (at.qt < a.nqt) {
         at.mw = kvalid ? a.masks[(bh * a.nqt + at.qt) * a.nb + ck] : 0ull;
         const int64_t row = at.qt * 64 + lane;
-        if (tid < 128)  // (rows past the end belong to no list: any finite value will do)
-          at.ld = (tid < 64 ? a.lse : a.delta)[bh * a.n + (row < a.n ? row : a.n - 1)];
+        if (tid < 128)  // (rows past the end belong to no list, but an infinity would be NaN)
+          at.ld = row < a.n ? (tid < 64 ? a.lse : a.delta)[bh * a.n + row] : 0.0f;
         break;
       }
     }

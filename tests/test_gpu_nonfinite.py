@@ -107,3 +107,42 @@ def test_prefill_value_of_infinity_in_the_last_row(cuda, dtype, d, hq, hkv, n, b
     tol = 1e-5 if dtype == torch.float32 else 2e-2
     same(out[..., rest], ref[..., rest], tol)
     same(out[:, :, n - 1], ref[:, :, n - 1], tol)
+
+
+# the same through the masked attention, forward and backward: an infinite value (a gradient) in the
+# last row makes the output (dV) infinite for the rows (keys) that meet it there
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hq,hkv,n,block", [(2, 1, 200, 64), (2, 2, 1000, 64), (4, 2, 150, 24)])
+def test_masked_attention_infinity_in_the_last_row(cuda, dtype, hq, hkv, n, block):
+    from ssa_amd import ssa_swap as S
+    rng = np.random.default_rng(n)
+    q, k, v, g = (WL.round_to(rng.standard_normal((1, h, n, 64)).astype(np.float32), dtype)
+                  for h in (hq, hkv, hkv, hq))
+    kn, ki = S.route_masked(*(WL.to_device(x, dtype, cuda) for x in (q, k)), block, 2, 1)
+    kn, ki = kn.cpu().numpy(), ki.cpu().numpy()
+    lists = np.empty((1, hq, n), dtype=object)
+    for at in np.ndindex(*lists.shape):
+        lists[at] = ki[at][:kn[at]].tolist()
+    tol = 1e-5 if dtype == torch.float32 else 2e-2
+    rest = [e for e in range(64) if e != 3]
+
+    def run(v, g):
+        t = [WL.to_device(x, dtype, cuda).requires_grad_(True) for x in (q, k, v)]
+        out = S.ssa_masked(*t, block, 2, 1)
+        return np_of(out), np_of(torch.autograd.grad(out, t, WL.to_device(g, dtype, cuda))[2])
+
+    out, dv = run(v, g)
+    bad = v.copy()
+    bad[:, :, n - 1, 3] = INF
+    got, _ = run(bad, g)
+    assert (got[:, :, n - 1, 3] == INF).all()
+    same(got[..., rest], out[..., rest], tol)
+    bad = g.copy()
+    bad[:, hq - 1, n - 1, 3] = INF
+    _, got = run(v, bad)
+    h = hkv - 1
+    seen = np.zeros(n, bool)  # the keys that the last row attends
+    for c in lists[0, hq - 1, n - 1]:
+        seen[c * block:(c + 1) * block] = True
+    assert (got[0, h, seen, 3] == INF).all()
+    same(got[0, :, :, rest], dv[0, :, :, rest], tol * max(1.0, np.abs(dv).max()))
