@@ -32,9 +32,10 @@ from .ssa_kernel import BLOCK, sparse_attention
 NEG = float("-inf")
 MAX_SEARCH = 1024   # search_k (staged, and committed after escalation) the route kernel takes
 MAX_QUOTA = 2048    # outliers kept per appended chunk
-# Largest block of scores route() has computed ahead of the search, 2 % of an MI355X's HBM (1024
-# query blocks against 20,000 rows take 80 MB); beyond it the search computes them row by row.
-SCORE_WORKSPACE_LIMIT = 6 << 30
+# Largest block of scores route() has computed ahead of the search: a chunk of 2048 query blocks
+# against 32,000 rows. More query blocks are routed in slices that fit; where not even one tile of
+# 64 fits, or the memory is not there, the search computes the scores row by row.
+SCORE_WORKSPACE_LIMIT = 256 << 20
 
 
 def _rows(x: torch.Tensor) -> torch.Tensor:
@@ -314,7 +315,7 @@ class CausalCascade:
         rounds = torch.zeros(nbq, dtype=torch.int32, device=dev)
         ix = self.index
         means = self.means
-        carry = 0
+        skmax = 0
         if ix is not None and certify and self.max_escalations > 0:
             # escalation carry: per query block the best keys of the lists probed so far, as many
             # as the last round's search_k
@@ -322,26 +323,44 @@ class CausalCascade:
             for _ in range(self.max_escalations):
                 sk = min(2 * sk, self.committed)
             skmax = max(min(sk0, self.committed), sk)
-            carry = -(-8 * nbq * skmax // 256) * 256
-        # the scores of the staged (and, before the index, the committed) means and the outliers
-        cols = [self.n_sub - self.committed, 0 if ix is not None else self.committed, self.n_out]
-        scores = 4 * nbq * sum(-(-c // 4) * 4 for c in cols)
-        ws_bytes = carry + (scores if scores <= SCORE_WORKSPACE_LIMIT else 0)
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
-        _lib.call("ssa_ccc_route", qr.data_ptr(), nbq, qb_start, self.dr,
-                  None if means is None else means.data_ptr(), self.committed, self.n_sub,
-                  self.spb, None if ix is None else ix.buf.data_ptr(),
-                  0 if ix is None else ix.n_cap, 0 if ix is None else ix.nlist,
-                  None if self.O is None else self.O.data_ptr(),
-                  None if self.O_parent is None else self.O_parent.data_ptr(), self.n_out,
-                  self.top_c, self.local, self.outlier_cap, self.search_k, sk0, self.nprobe,
-                  self.escalate_factor, self.max_escalations, 1 if certify else 0,
-                  float(self.cert_margin), kv_num.data_ptr(), kv_idx.data_ptr(), W,
-                  cert.data_ptr(), rounds.data_ptr(), None if ws is None else ws.data_ptr(),
-                  ws_bytes, _lib.stream_of(qr))
+        ws, step = self._route_workspace(nbq, 8 * skmax, dev)
+        for a in range(0, nbq, step):
+            _lib.call("ssa_ccc_route", qr.data_ptr() + 4 * self.dr * a, min(step, nbq - a),
+                      qb_start + a, self.dr, None if means is None else means.data_ptr(),
+                      self.committed, self.n_sub, self.spb,
+                      None if ix is None else ix.buf.data_ptr(),
+                      0 if ix is None else ix.n_cap, 0 if ix is None else ix.nlist,
+                      None if self.O is None else self.O.data_ptr(),
+                      None if self.O_parent is None else self.O_parent.data_ptr(), self.n_out,
+                      self.top_c, self.local, self.outlier_cap, self.search_k, sk0, self.nprobe,
+                      self.escalate_factor, self.max_escalations, 1 if certify else 0,
+                      float(self.cert_margin), kv_num.data_ptr() + 4 * a,
+                      kv_idx.data_ptr() + 4 * W * a, W, cert.data_ptr() + a,
+                      rounds.data_ptr() + 4 * a,
+                      None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(),
+                      _lib.stream_of(qr))
         stats = {"nbq": nbq, "rounds": rounds,
                  "cert_rate": float(cert.float().mean()) if certify and nbq else None}
         return kv_num, kv_idx, (cert.bool() if certify else None), stats
+
+    def _route_workspace(self, nbq, carry, dev):
+        """(workspace or None, query blocks a call) for nbq query blocks of `carry` bytes each and
+        their scores against the staged (and, before the index, the committed) means and the
+        outliers."""
+        cols = [self.n_sub - self.committed, 0 if self.index is not None else self.committed,
+                self.n_out]
+        scores = 4 * sum(-(-c // 4) * 4 for c in cols)
+        step = nbq
+        if nbq * scores > SCORE_WORKSPACE_LIMIT:
+            step = SCORE_WORKSPACE_LIMIT // scores // 64 * 64
+        if step and scores:
+            try:
+                return torch.empty(-(-carry * step // 256) * 256 + scores * step,
+                                   dtype=torch.uint8, device=dev), step
+            except torch.OutOfMemoryError:
+                pass
+        ws = torch.empty(carry * nbq, dtype=torch.uint8, device=dev) if carry else None
+        return ws, max(nbq, 1)
 
     # -- decode ----------------------------------------------------------------------------------
 

@@ -1,0 +1,80 @@
+"""The cascade route's workspace: bounded, routed in slices where the scores need more, and no
+scores where the memory is not there. Selections equal the row-by-row search's in every case."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def cascade(cuda, seed, blocks, d, **kw):
+    from ssa_amd import cascade_router as C
+    g = torch.Generator(device=cuda).manual_seed(seed)
+    cc = C.CausalCascade(d, search_k=48, **kw)
+    for n in blocks:
+        cc.append(torch.randn(n * 128, d, device=cuda, generator=g).half())
+    return cc, g
+
+
+def routed(cc, q, first, certify):
+    """(block lists, certificates, rounds) of one route call, on the host."""
+    kn, ki, cert, st = cc.route(q, first * 128, certify=certify)
+    kn, ki = kn.cpu().numpy(), ki.cpu().numpy()
+    return ([ki[i, :kn[i]].tolist() for i in range(len(kn))],
+            None if cert is None else cert.cpu().numpy().tolist(),
+            st["rounds"].cpu().numpy().tolist())
+
+
+def test_workspace_stays_bounded(cuda, monkeypatch):
+    """2048 query blocks against 65,664 rows: 0.5 GB of scores in one piece."""
+    from ssa_amd import cascade_router as C
+    cc, g = cascade(cuda, 1, (64, 16352), 32, outlier_rate=5e-4)
+    q = torch.randn(2048 * 128, 32, device=cuda, generator=g).half()
+    torch.cuda.synchronize()
+    base = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    got = routed(cc, q, 16416 - 2048, False)
+    assert torch.cuda.max_memory_allocated() - base < 300 << 20
+    monkeypatch.setattr(C, "SCORE_WORKSPACE_LIMIT", 0)
+    assert routed(cc, q, 16416 - 2048, False) == got
+
+
+# slices of one score tile and of two, a remainder of one query block; with an index the slices
+# share the escalation carry
+@pytest.mark.parametrize("indexed", [False, True])
+@pytest.mark.parametrize("nbq,tiles", [(129, 1), (200, 2), (64, 1), (63, 0)])
+def test_slices_select_the_same(cuda, monkeypatch, indexed, nbq, tiles):
+    from ssa_amd import cascade_router as C
+    kw = dict(nlist=40, nprobe=2) if indexed else {}
+    from_blocks = (700, 300)
+    cc, g = cascade(cuda, nbq, (), 64, **kw)
+    cc.build_threshold = 1000 if indexed else 1 << 30
+    for n in from_blocks:
+        cc.append(torch.randn(n * 128, 64, device=cuda, generator=g).half())
+    assert (cc.index is not None) == indexed
+    q = torch.randn(nbq * 128, 64, device=cuda, generator=g).half()
+    ref = routed(cc, q, 1000 - nbq, True)
+    rows = (cc.n_sub - cc.committed + 3) // 4 * 4 + (cc.n_out + 3) // 4 * 4
+    rows += 0 if indexed else (cc.committed + 3) // 4 * 4
+    monkeypatch.setattr(C, "SCORE_WORKSPACE_LIMIT", (64 * tiles + 1) * 4 * rows)
+    assert cc._route_workspace(nbq, 0, cuda)[1] == (min(nbq, 64 * tiles) if tiles else nbq)
+    assert routed(cc, q, 1000 - nbq, True) == ref
+
+
+def test_no_memory_for_the_scores(cuda, monkeypatch):
+    """The allocation of the scores fails: the call routes with the carry alone."""
+    cc, g = cascade(cuda, 3, (), 64, nlist=40, nprobe=2)
+    cc.build_threshold = 1000
+    for n in (700, 300):
+        cc.append(torch.randn(n * 128, 64, device=cuda, generator=g).half())
+    q = torch.randn(100 * 128, 64, device=cuda, generator=g).half()
+    ref = routed(cc, q, 900, True)
+    empty, tried = torch.empty, []
+
+    def short(*a, **k):
+        if k.get("dtype") == torch.uint8 and a[0] > 400_000:
+            tried.append(a[0])
+            raise torch.OutOfMemoryError("no memory")
+        return empty(*a, **k)
+    monkeypatch.setattr(torch, "empty", short)
+    got = routed(cc, q, 900, True)
+    assert tried and got == ref
