@@ -293,8 +293,8 @@ int ssa_tree_pack(const int32_t* sel, int64_t rows, int64_t nb, int64_t tc, int6
  *   largest search_k a round uses (min(search_k, committed), doubled per escalation up to
  *   committed): each round keeps the skmax best committed keys of the lists probed so far there,
  *   so a later round scans only the lists it adds; otherwise ws may be NULL. Room for the scores
- *   after the carry (rounded up to 256 bytes; ws 16-byte aligned) lets the call compute them first,
- *   a row read once per 64 query blocks (the same values): nbq * 4 * (R4(n_sub - committed) +
+ *   after the carry (rounded up to 256 bytes; ws 16-byte aligned) lets the call compute them first
+ *   where that is faster, a row read once per 64 query blocks (the same values): nbq * 4 * (R4(n_sub - committed) +
  *   (without an index) R4(committed) + R4(n_out)) bytes, R4 rounding up to a multiple of 4.
  */
 size_t ssa_ccc_index_size(int64_t n_cap, int64_t nlist, int64_t d);

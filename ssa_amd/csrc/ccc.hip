@@ -580,6 +580,17 @@ struct CccRouteArgs {
 // prefill (8 chunks of 1024 query blocks, 181 cells): route kernels 2960 us before; 1463 us and 335
 // us of scoring (fp64 fma rate: 25 us for 1024 x 12,288 x 64) with the scores read from memory.
 constexpr int kScoreQ = 64, kScoreC = 128, kScoreD = 32;
+
+// Whether ccc_score_kernel runs ahead of the search (`launches` of it, `rows` scores a query block):
+// a launch costs about 8 us, and what it saves grows with the rows and, as the row-by-row search
+// fills the chip (3 workgroups a CU), with the query blocks. Route call ahead / row by row, d 64:
+// 1 query block, 2 launches: 1276 rows 72 / 60 us, 3192 83 / 82, 5320 83 / 95; 3 launches: 1238 rows
+// 80 / 58, 4952 94 / 95, 10,320 97 / 130; 300 query blocks, 2 launches: 2128 rows 85 / 81, 3192 91 / 99;
+// 512: 1782 rows 90 / 89; 1024 (a second wave of workgroups row by row): 824 rows 94 / 110. The line
+// moves to 0.8 of these rows at d 128 and 256 and to 1.3 at d 32.
+inline bool scores_ahead(int64_t nbq, int64_t rows, int launches) {
+  return nbq > 768 || rows * (nbq + 600) >= launches * 960000ll;
+}
 __global__ __launch_bounds__(256) void ccc_score_kernel(const float* __restrict__ qr, int64_t nbq,
                                                         const float* __restrict__ x, int64_t m,
                                                         int64_t d, int64_t j0, int64_t spb,
@@ -1273,14 +1284,15 @@ extern "C" int ssa_ccc_route(const float* qr, int64_t nbq, int64_t qb_start, int
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
   const size_t lds = ssa::CccRouteLds(a).bytes();
-  // precomputed scores, where the workspace has room for them after the carry
+  // precomputed scores, where they pay and the workspace has room for them after the carry
   const int64_t nsr = ks > 0 ? (ns + 3) & ~int64_t(3) : 0;
   const int64_t ncr = index == nullptr ? (committed + 3) & ~int64_t(3) : 0;
   const int64_t nor = ocap > 0 ? (n_out + 3) & ~int64_t(3) : 0;
   const size_t at = (carry_bytes + 255) & ~size_t(255);
   const size_t sbytes = size_t(nbq) * size_t(nsr + ncr + nor) * 4;
   const int64_t qtiles = (nbq + ssa::kScoreQ - 1) / ssa::kScoreQ;
-  if (sbytes == 0 || ws == nullptr || ws_bytes < at + sbytes || qtiles > 65535 ||
+  if (sbytes == 0 || !ssa::scores_ahead(nbq, nsr + ncr + nor, (nsr > 0) + (ncr > 0) + (nor > 0)) ||
+      ws == nullptr || ws_bytes < at + sbytes || qtiles > 65535 ||
       (reinterpret_cast<uintptr_t>(ws) & 15u) != 0) {
     ssa::ccc_route_kernel<false><<<(unsigned)nbq, 256, lds, st>>>(a);
     return ssa::launch_status("ccc_route_kernel");

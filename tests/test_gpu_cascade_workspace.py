@@ -78,3 +78,34 @@ def test_no_memory_for_the_scores(cuda, monkeypatch):
     monkeypatch.setattr(torch, "empty", short)
     got = routed(cc, q, 900, True)
     assert tried and got == ref
+
+
+# short contexts, few query blocks: the scores ahead cost more launches than they save
+@pytest.mark.parametrize("d,blocks,nbq,indexed,ahead", [
+    (64, (30, 30), 8, False, False), (64, (150, 150), 1, False, False),
+    (128, (300, 300), 64, True, False), (64, (1300, 1300), 1, False, True),
+    (96, (700, 700), 1, False, True), (32, (550, 550), 129, False, True),
+    (256, (300, 700), 300, True, True), (32, (700, 1100), 130, True, True),
+    (64, (300, 300), 800, False, True)])
+def test_scores_ahead_only_where_they_pay(cuda, monkeypatch, d, blocks, nbq, indexed, ahead):
+    """The workspace shows whether the scores were written; the selection is the same."""
+    from ssa_amd import cascade_router as C
+    cc, g = cascade(cuda, d, (), d, **(dict(nlist=40, nprobe=2) if indexed else {}))
+    cc.build_threshold = 1000 if indexed else 1 << 30
+    for n in blocks:
+        cc.append(torch.randn(n * 128, d, device=cuda, generator=g).half())
+    assert (cc.index is not None) == indexed
+    q = torch.randn(nbq * 128, d, device=cuda, generator=g).half()
+    first = max(sum(blocks) - nbq, 200)
+    empty, made = torch.empty, []
+
+    def marked(*a, **k):
+        t = empty(*a, **k)
+        if k.get("dtype") == torch.uint8:
+            made.append(t.fill_(0xA5))
+        return t
+    monkeypatch.setattr(torch, "empty", marked)
+    got = routed(cc, q, first, False)
+    assert len(made) == 1 and bool((made[0] != 0xA5).any()) == ahead
+    monkeypatch.setattr(C, "SCORE_WORKSPACE_LIMIT", 0)
+    assert routed(cc, q, first, False) == got
