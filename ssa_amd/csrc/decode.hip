@@ -1663,7 +1663,17 @@ int decode_step_impl(const void* q, const void* k_new, const void* v_new, void* 
     f.kv_num = kv_num;
     f.kv_idx = kv_idx;
     f.lseg = attend_segment_log2(f.nchunk, 8);
-    const size_t alds = ((size_t)8 << f.lseg) * 8;  // (key, block) per entry
+    size_t alds = ((size_t)8 << f.lseg) * 8;  // (key, block) per entry
+    // bf16 at head dim 64, blocks of more than 128 (a key row per lane: two workgroups a CU evict
+    // each other's lines): a grid of just two workgroups a CU is faster one after the other, as
+    // LDS that lets only one onto a CU makes it. Step times together / one after the other: 512
+    // workgroups, block 256 52.2 / 48.7 us, 384 63.2 / 57.5, 512 74.7 / 64.7; 560, block 256 58 /
+    // 61, 512 90 / 84; 480, block 256 47.6 / 51.1, 512 62.1 / 65.1; 768, block 256 67 / 70, 512 92
+    // / 93. (fp16 takes a CU alone by its registers.)
+    const int64_t attend_wgs = f.ngroups * B * Hq;
+    if (dtype == SSA_BF16 && d == 64 && block > 128 && attend_wgs > 480 &&
+        attend_wgs <= block + 256)
+      alds = alds < 55000 ? 55000 : alds;
     const dim3 g1((unsigned)nchunk, (unsigned)(B * Hkv)), g2((unsigned)f.ngroups, (unsigned)(B * Hq));
 #define SSA_FUSED_ROUTE(DT, NW, NWT)                                                              \
   do {                                                                                            \
