@@ -830,9 +830,9 @@ __device__ inline void attend_group(const FusedStep& f, const DecodeParams& p, i
                                     int64_t group) {
   constexpr int NT = NWA * 64, SPW = NWA / HALVES;
   // survivors of the merge, a segment per wave: as many entries as this step's chunk lists hold
-  // (attend_lds), not the most there can be (64 KB, which left one workgroup on a CU whatever the
-  // context). LONG (the most, more than 64 chunks): a fixed array, which the merge addresses
-  // faster: 25.3 us a step against 25.7 at 8192 blocks
+  // (dynamic LDS), not the most there can be (64 KB, which left one workgroup on a CU whatever the
+  // context). LONG: a fixed array of the most, which the merge addresses faster: 25.3 us a step
+  // against 25.7 at 8192 blocks (when: decode_step_impl)
   extern __shared__ unsigned int dyn_lds[];
   __shared__ unsigned int held[LONG ? 2 * kDSurv : 1];
   const int lseg = LONG ? 10 : f.lseg;
@@ -1663,17 +1663,19 @@ int decode_step_impl(const void* q, const void* k_new, const void* v_new, void* 
     f.kv_num = kv_num;
     f.kv_idx = kv_idx;
     f.lseg = attend_segment_log2(f.nchunk, 8);
-    size_t alds = ((size_t)8 << f.lseg) * 8;  // (key, block) per entry
-    // bf16 at head dim 64, blocks of more than 128 (a key row per lane: two workgroups a CU evict
-    // each other's lines): a grid of just two workgroups a CU is faster one after the other, as
-    // LDS that lets only one onto a CU makes it. Step times together / one after the other: 512
-    // workgroups, block 256 52.2 / 48.7 us, 384 63.2 / 57.5, 512 74.7 / 64.7; 560, block 256 58 /
+    const size_t alds = ((size_t)8 << f.lseg) * 8;  // (key, block) per entry
+    // The fixed array (one workgroup a CU, constant addresses in the merge) is the better one past
+    // 64 chunks (see attend_group), where the grid puts at most one workgroup on a CU anyway, and
+    // (bf16, head dim 64, blocks of more than 128: a key row per lane, two workgroups a CU evict
+    // each other's lines) where it is just two workgroups a CU. Step times, sized by the step /
+    // fixed, head dim 64: 128-256 workgroups, block 64 and 128 21.9 / 21.4 us, 23.8 / 23.3; 320
+    // 31.0 / 33.7; 512, block 256 52.2 / 48.7, 384 63.2 / 57.5, 512 74.7 / 64.7; 560, block 256 58 /
     // 61, 512 90 / 84; 480, block 256 47.6 / 51.1, 512 62.1 / 65.1; 768, block 256 67 / 70, 512 92
-    // / 93. (fp16 takes a CU alone by its registers.)
-    const int64_t attend_wgs = f.ngroups * B * Hq;
-    if (dtype == SSA_BF16 && d == 64 && block > 128 && attend_wgs > 480 &&
-        attend_wgs <= block + 256)
-      alds = alds < 55000 ? 55000 : alds;
+    // / 93.
+    const int64_t wgs = f.ngroups * B * Hq;
+    const bool fixed = f.lseg == 10 || wgs <= 256 ||
+                       (dtype == SSA_BF16 && d == 64 && block > 128 && wgs > 480 &&
+                        wgs <= block + 256);
     const dim3 g1((unsigned)nchunk, (unsigned)(B * Hkv)), g2((unsigned)f.ngroups, (unsigned)(B * Hq));
 #define SSA_FUSED_ROUTE(DT, NW, NWT)                                                              \
   do {                                                                                            \
@@ -1690,7 +1692,7 @@ int decode_step_impl(const void* q, const void* k_new, const void* v_new, void* 
     if (w && d == 128 && f.lseg < 10)                                                             \
       decode_attend_fused_kernel<DT, w, false><<<g2, 512, alds, st>>>(f, p);                      \
     else if (w && d == 128) decode_attend_fused_kernel<DT, w, true><<<g2, 512, 0, st>>>(f, p);    \
-    else if (f.lseg < 10) decode_attend_fused_kernel<DT, false, false><<<g2, 512, alds, st>>>(f, p); \
+    else if (!fixed) decode_attend_fused_kernel<DT, false, false><<<g2, 512, alds, st>>>(f, p);     \
     else decode_attend_fused_kernel<DT, false, true><<<g2, 512, 0, st>>>(f, p);                   \
   } while (0)
     switch (dtype) {

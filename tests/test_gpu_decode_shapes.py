@@ -43,3 +43,15 @@ def check_steps(cuda, dtype, B, hq, hkv, d, block, n, top_c, steps=2, rows=((0, 
 @pytest.mark.parametrize("block", [256, 512])
 def test_decode_step_two_workgroups_a_cu(cuda, B, hq, hkv, top_c, block):
     check_steps(cuda, torch.bfloat16, B, hq, hkv, 64, block, 6 * block + block // 3, top_c)
+
+
+# the merge's segments: chunk lists that fill one, two, four and eight of a wave's 64-entry lists (up
+# to 64 chunks) and the fixed array (more), with grids of more than 256 workgroups; head dim 64 also
+# with a grid of one workgroup a CU, which takes the fixed array
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("d,hq,nblocks,top_c", [
+    (128, 32, 60, 40), (128, 32, 700, 64), (128, 32, 1500, 64), (128, 32, 3500, 64),
+    (128, 32, 4200, 64), (64, 32, 60, 40), (64, 32, 700, 64), (64, 32, 1500, 64),
+    (64, 32, 3500, 64), (64, 4, 3500, 64)])
+def test_decode_step_merge_segments(cuda, dtype, d, hq, nblocks, top_c):
+    check_steps(cuda, dtype, 1, hq, 2, d, 16, 16 * nblocks + 5, top_c)
