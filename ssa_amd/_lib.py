@@ -165,10 +165,16 @@ def ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+# the raw handle without a torch.cuda.Stream around it, which cost as much as the launch (a private
+# function: a torch build without it takes the public way)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_of(t: torch.Tensor) -> int:
-    """The current HIP stream of t's device as a raw handle (without a torch.cuda.Stream around it,
-    which cost as much as the launch)."""
-    return torch._C._cuda_getCurrentRawStream(t.device.index)
+    """The current HIP stream of t's device as a raw handle."""
+    if _raw_stream is None:
+        return torch.cuda.current_stream(t.device).cuda_stream
+    return _raw_stream(t.device.index)
 
 
 def i64_array(values) -> ctypes.Array:

@@ -181,3 +181,17 @@ def test_custom_op_fake_shapes():
     o = ops.decode_step(qd, kn, kn, kc, kc, mus, mus, num, idx, None, 100, 128, 64, 0.0, 1, 1.0,
                         0.125)
     assert o.shape == (1, 14, 64)
+
+
+def test_stream_handle_without_the_raw_getter(monkeypatch):
+    """A torch build without the private raw-handle getter: the stream comes from torch.cuda."""
+    from importlib import util
+    from types import SimpleNamespace as NS
+
+    import torch
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda dev: NS(cuda_stream=77 + dev.index))
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+    spec = util.spec_from_file_location("ssa_amd._lib_copy", _lib.__file__)
+    copy = util.module_from_spec(spec)
+    spec.loader.exec_module(copy)
+    assert copy.stream_of(NS(device=NS(index=1))) == 78
