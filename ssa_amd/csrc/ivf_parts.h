@@ -135,6 +135,7 @@ __device__ unsigned long long block_kth_largest(const unsigned long long* keys, 
 // its rows. d 64: 8192 means, 90 centroids 20 -> 6.6 us (the matrix rate alone: 1.3); 8192 to 32,768
 // means, 181 centroids 23 -> 11.5 on average. What is left is the launch and one wait for the rows.
 typedef double ivf_f64x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));  // (a caller's centroids)
 
 // Element e of the lanes of quarter q (lane / 16) <-> element q of the lanes of quarter e.
 __device__ inline f32x4 quarter_transpose(const f32x4& x) {
@@ -181,7 +182,7 @@ __global__ __launch_bounds__(256) void ivf_score_kernel(
   auto load = [&](int tile, f32x4* a) {  // (rows past the last centroid re-read it: discarded)
     const int64_t c = 16 * (int64_t)tile + col < nlist ? 16 * (int64_t)tile + col : nlist - 1;
 #pragma unroll
-    for (int v = 0; v < NV; ++v) a[v] = *reinterpret_cast<const f32x4*>(cb + c * D + 16 * v);
+    for (int v = 0; v < NV; ++v) a[v] = *reinterpret_cast<const f32x4_u*>(cb + c * D + 16 * v);
   };
   unsigned long long best[2] = {0ull, 0ull};
   f32x4 a[NV];

@@ -109,3 +109,26 @@ def test_scores_ahead_only_where_they_pay(cuda, monkeypatch, d, blocks, nbq, ind
     assert len(made) == 1 and bool((made[0] != 0xA5).any()) == ahead
     monkeypatch.setattr(C, "SCORE_WORKSPACE_LIMIT", 0)
     assert routed(cc, q, first, False) == got
+
+
+def test_centroids_at_any_float(cuda):
+    """Assignment and k-means read a caller's centroids at 4-byte alignment."""
+    from ssa_amd import _lib
+    g = torch.Generator(device=cuda).manual_seed(5)
+    n, nlist, d = 300, 37, 96
+    x = torch.randn(n, d, device=cuda, generator=g)
+    c = torch.randn(nlist, d, device=cuda, generator=g)
+    ws = torch.empty(int(_lib.query("ssa_ccc_index_size", n, nlist, d)), dtype=torch.uint8,
+                     device=cuda)
+    res = []
+    for shift in (0, 1, 2, 3):
+        buf = torch.empty(nlist * d + 4, device=cuda)
+        cent = buf[shift:shift + nlist * d]
+        cent.copy_(c.view(-1))
+        assign = torch.empty(n, dtype=torch.int32, device=cuda)
+        _lib.call("ssa_ccc_assign", x.data_ptr(), n, d, cent.data_ptr(), nlist, assign.data_ptr(),
+                  ws.data_ptr(), ws.numel(), _lib.stream_of(x))
+        _lib.call("ssa_ccc_kmeans", x.data_ptr(), n, d, nlist, 2, 1, cent.data_ptr(),
+                  ws.data_ptr(), ws.numel(), _lib.stream_of(x))
+        res.append((assign.tolist(), cent.tolist()))
+    assert all(r == res[0] for r in res[1:])
