@@ -334,10 +334,13 @@ int ssa_ccc_route(const float* qr, int64_t nbq, int64_t qb_start, int64_t d, con
  * softmax(scale * q.k) in fp32; out has q's dtype. strides[12] = q(b,h,n), k(b,h,n), v(b,h,n),
  * out(b,h,n) in elements. lse (B, Hq, n) fp32 natural-log sum-exp, may be NULL.
  * dtype: SSA_BF16 / SSA_F16 (MFMA, d = 64, 128, 256 or 512) or SSA_F32 (d = 64). block: 64 or a
- * multiple of 128. At d = 512 the four waves of a workgroup split the head dim over 32 query
- * rows and sum their partial scores in wave order (the same order for every row).
+ * multiple of 128. At d = 512 calls of fewer than 96 groups of 128 query rows split the head dim
+ * over the four waves of a workgroup of 32 rows, which sum their partial scores in wave order (the
+ * same order for every row); from 96 groups on a wave owns 16 rows of a workgroup of 64 or 128.
  * The 16-bit paths read V transposed, (B, Hkv, d, n_pad) with n_pad = ceil(n/block)*block, from
- * the workspace (ssa_sparse_attn_workspace_size() bytes). flags = 0: the call first writes V^T
+ * the workspace (ssa_sparse_attn_workspace_size() bytes), but for d = 512 from 96 groups on, which
+ * reads v itself (the workspace is required all the same and stays untouched, and a V^T that it
+ * holds is not read: v must be the one it was made from). flags = 0: the call first writes V^T
  * there itself; flags = SSA_ATTN_VT_READY: the workspace already holds V^T of this v (from
  * ssa_transpose_v), e.g. kept resident across calls. After V^T the workspace holds per-call state
  * (d = 64: for bf16 an fp16 copy of K, the largest squared key norm of every 64-key tile, one

@@ -60,11 +60,6 @@ struct SwapArgs {
   float scale, scale_log2;
 };
 
-template <int DT>
-__host__ __device__ constexpr int dtype_size_dev() {
-  return DT == SSA_F32 ? 4 : 2;
-}
-
 __device__ inline f32x16 mfma(float a, float b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }

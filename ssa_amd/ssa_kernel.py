@@ -255,7 +255,8 @@ def sparse_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, kv_num: 
 
     q (B, Hq, n, d); k, v (B, Hkv, n, d); kv_num (B, Hq, nb); kv_idx (B, Hq, nb, W).
     `out` may be any (B, Hq, n, d) view with a contiguous last dim (e.g. a transpose of a
-    (B, n, Hq, d) buffer). `vt` is an optional V^T from transpose_v(v, block).
+    (B, n, Hq, d) buffer). `vt` is an optional V^T from transpose_v(v, block) of this v (head dim
+    512 from 96 groups of 128 query rows on reads v itself and makes no use of it).
     Every query block walks its key blocks in list order (bit-identical outputs across calls).
     `rotate` (16-bit, head dim 64, lists of <= 128 entries; ignored under
     torch.use_deterministic_algorithms(True)): each workgroup starts its walk at a position taken

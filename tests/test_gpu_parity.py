@@ -1169,8 +1169,8 @@ def _lse64(q, k, kv_num, kv_idx, block, scale):
 def test_tiled_prefill_wide_head_dims_match_oracle(cuda, d, dtype, block):
     """The tiled MFMA prefill kernels at head dims 128 and 256 (4 waves x 32 query rows per
     128-row query tile, 2 waves for block 64; 64-key sub-tiles, 32-key at head dim 256; exact
-    running-max softmax) and 512 (sparse_attn_wide_kernel: 4 waves split the head dim over one
-    32-row query group, 32-key sub-tiles): ragged n, GQA 3:1, the oracle router's lists (budget
+    running-max softmax) and 512 (sparse_attn_wide_kernel, which serves calls this small: 4 waves
+    split the head dim over one 32-row query group, 32-key sub-tiles): ragged n, GQA 3:1, the oracle router's lists (budget
     0.4 + local 1), every query row against the oracle within 2e-2, lse within 2^-8 of the
     float64 log-sum-exp (the row sum adds each P after rounding it to the 16-bit input type, a
     relative error of at most 2^-9 per term, so |d lse| <= 2^-9 plus fp32 accumulation), and a

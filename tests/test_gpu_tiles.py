@@ -1,5 +1,8 @@
 """GPU kernels at the sizes where their tilings change or leave remainders, against the CPU oracle
 (float64)."""
+import re
+from pathlib import Path
+
 import numpy as np
 import pytest
 import torch
@@ -50,8 +53,8 @@ def test_fp32_attention_tiles_match_oracle(cuda, hq, hkv, n, block, W):
     assert abs(float(lse[0, h, n - 1]) - np.log(np.exp(s).sum())) < 1e-5
 
 
-# head dim 512: fewer than 96 groups of 128 rows (32-row workgroups), 4-wave groups (also every
-# block of 64), 8-wave groups; lengths that end inside a wave's rows and inside a 32-key sub-tile
+# head dim 512: fewer than 96 groups of 128 rows (32-row workgroups, also at block 64), 4-wave
+# groups, 8-wave groups; lengths that end inside a wave's rows and inside a 32-key sub-tile
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("hq,hkv,n,block,W", [(2, 1, 300, 64, 3), (16, 4, 797, 128, 4),
                                               (32, 32, 261, 64, 5), (24, 8, 1043, 256, 3),
@@ -73,6 +76,34 @@ def test_d512_attention_tiles_match_oracle(cuda, dtype, hq, hkv, n, block, W):
     assert np.abs(np_of(out)[:, heads] - ref[:, heads]).max() < 2e-2
     none = ~np.isfinite(ref[0, 0]).all(-1) | (ref[0, 0] == 0).all(-1)
     assert (torch.isneginf(lse[0, 0]).cpu().numpy() == none).all()
+
+
+# head dim 512 from 96 groups of 128 rows on, which reads V itself: block 64 (4-wave groups), 4- and
+# 8-wave groups, also with a V^T or a prepared workspace, whose V^T such a call does not read
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hq,hkv,n,block,W", [(48, 8, 261, 64, 3), (16, 4, 850, 128, 3),
+                                              (24, 8, 1043, 256, 3)])
+def test_d512_attention_given_workspaces(cuda, dtype, hq, hkv, n, block, W):
+    """2e-2: the bar of every 16-bit attention test; the given workspaces change no bit."""
+    src = (Path(__file__).resolve().parents[1] / "ssa_amd/csrc/attn.hip").read_text()
+    nb = -(-n // block)
+    least = int(re.search(r"kWide16Min = (\d+)", src).group(1))
+    assert nb * block // 64 * hq // 2 >= least, "the case no longer reaches the 128-row kernel"
+    rng = np.random.default_rng(n)
+    q, k, v = (WL.round_to(rng.standard_normal((1, h, n, 512)).astype(np.float32), dtype)
+               for h in (hq, hkv, hkv))
+    kv_num, kv_idx = random_lists(rng, hq, nb, min(W, nb))
+    qt, kt, vt = (WL.to_device(a, dtype, cuda) for a in (q, k, v))
+    num, idx = torch.from_numpy(kv_num).to(cuda), torch.from_numpy(kv_idx).to(cuda)
+    out = K.sparse_attention(qt, kt, vt, num, idx, block)
+    heads = [0, hq - 1]
+    ref = O.sparse_attention(q, k, v, kv_num, kv_idx, block, heads=heads)
+    assert np.abs(np_of(out)[:, heads] - ref[:, heads]).max() < 2e-2
+    given = K.sparse_attention(qt, kt, vt, num, idx, block, vt=K.transpose_v(vt, block))
+    assert torch.equal(given, out)
+    given = K.sparse_attention(qt, kt, vt, num, idx, block,
+                               prepared=K.prepare_attention(kt, vt, block))
+    assert torch.equal(given, out)
 
 
 # cascade route: query blocks and rows that fill no 64 x 128 score tile, and candidates in rising
@@ -187,8 +218,9 @@ def test_masked_attention_tiles_match_oracle(cuda, dtype, hq, hkv, n, block, top
 
 
 # routed decode step: head dim 128 over parts of a block of less, exactly and more than 32 keys, the
-# new token first and last in its block; contexts whose chunk lists fill one, two and four segments
-# and all of the longest (more than 64 chunks: 4200 blocks), at head dim 64 too
+# new token first and last in its block; contexts of one chunk list, of one and of two a wave and
+# of the most (more than 64 chunks: 4200 blocks), at head dim 64 too (test_gpu_decode_shapes.py:
+# the lengths between)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("d,block,n,top_c", [(128, 16, 33, 2), (128, 64, 640, 4),
                                              (128, 512, 1800, 2), (128, 128, 131072, 8),
